@@ -306,7 +306,8 @@ __host__ __device__ inline uint32_t cell_key(int cx, int cy, int cz) {
 }
 // Cell coordinate of one axis (src/neighbor/verlet_list.cu:67-72)
 __device__ inline int cell_coord(float x, float inv_cs, int nx) {
-    int c = (int)floorf(x * inv_cs);
+    const int c = (int)floorf(x * inv_cs);
+    if ((unsigned)c < (unsigned)nx) return c;  // every wrapped position but one on the upper bound
     return ((c % nx) + nx) % nx;
 }
 

@@ -745,10 +745,6 @@ __device__ inline int wrap_cell(int c, int o, int nx) {
     return c;
 }
 
-// Appends the candidates of mask m (bit k: slot q0 + k) in slot order,
-// skipping the atom itself and its bonded partners.  Entry k is stored as
-// ebase + k (a staged index or a slot) and, with `used`, marks used[ebase + k].
-// W16 rows hold 16-bit entries (replicas of at most 65536 slots), others 32-bit.
 // The bits of candidates q0 + k that are the atom itself or a bonded partner.
 __device__ __forceinline__ unsigned excluded_mask(unsigned m, int q0, int i, const int (&ex)[4], int nb, int bcap,
                                                   const FMD_GLOBAL int* bt) {
@@ -762,41 +758,31 @@ __device__ __forceinline__ unsigned excluded_mask(unsigned m, int q0, int i, con
     return m & x;
 }
 
-template <bool W16>
-__device__ __forceinline__ void append_chunk(unsigned m, int q0, int i, const int (&ex)[4], int nb, int bcap,
-                                             const FMD_GLOBAL int* bt, FMD_GLOBAL int* out,
-                                             FMD_GLOBAL unsigned short* out16, int kcap, int& cnt, int ebase,
-                                             unsigned char* used) {
-    m &= ~excluded_mask(m, q0, i, ex, nb, bcap, bt);
-    // one pass per set bit, lowest first: a wave runs as many passes as its
-    // fullest lane has pairs in the chunk (about 4 of 8)
-    while (m) {
-        const int k = __builtin_ctz(m);
-        m &= m - 1u;
-        if (cnt < kcap) {
-            if (W16) out16[cnt * kTile] = (unsigned short)(ebase + k);
-            else out[cnt * kTile] = ebase + k;
-            if (used) used[ebase + k] = 1;
-        }
-        cnt++;
-    }
-}
-
-// One chunk of kBuildChunk candidates (slots q0 + k, k < n) by the reference
-// FP32 distance: the tests give a bit mask, then the set bits are appended.
+// One chunk of kBuildChunk candidates (slots q0 + k, k < n) of the global scan
+// by the reference FP32 distance: the tests give a bit mask, then the set bits
+// are appended in slot order, skipping the atom itself and its bonded partners.
+// W16 rows hold 16-bit entries (replicas of at most 65536 slots), others 32-bit.
 template <bool W16>
 __device__ __forceinline__ void build_chunk(const float4 (&pj)[kBuildChunk], int q0, int n, int i, float4 pi,
                                             float L, float invL, float rcs2, const int (&ex)[4], int nb,
                                             int bcap, const FMD_GLOBAL int* bt, FMD_GLOBAL int* out,
-                                            FMD_GLOBAL unsigned short* out16, int kcap, int& cnt, int ebase,
-                                            unsigned char* used) {
+                                            FMD_GLOBAL unsigned short* out16, int kcap, int& cnt) {
     unsigned m = 0;
 #pragma unroll
     for (int k = 0; k < kBuildChunk; k++) {
         const float r2 = dist2_ref(pi, pj[k], L, invL);  // every k: no per-candidate branch
         m |= ((k < n) & (r2 < rcs2)) ? (1u << k) : 0u;
     }
-    append_chunk<W16>(m, q0, i, ex, nb, bcap, bt, out, out16, kcap, cnt, ebase, used);
+    m &= ~excluded_mask(m, q0, i, ex, nb, bcap, bt);
+    while (m) {
+        const int k = __builtin_ctz(m);
+        m &= m - 1u;
+        if (cnt < kcap) {
+            if (W16) out16[cnt * kTile] = (unsigned short)(q0 + k);
+            else out[cnt * kTile] = q0 + k;
+        }
+        cnt++;
+    }
 }
 
 // The same decision with a coarse fixed-point prefilter.  The staged
@@ -826,174 +812,110 @@ __device__ __forceinline__ unsigned coarse_xy(int4 p) {
     return ((unsigned)p.x >> 16) | ((unsigned)p.y & 0xFFFF0000u);
 }
 __device__ __forceinline__ unsigned coarse_z(int4 p) { return (unsigned)p.z >> 16; }
-// The lowest r set bits of m (none for r <= 0).
-__device__ inline unsigned lowest_bits(unsigned m, int r) {
-    unsigned keep = 0u;
-    for (int j = 0; j < r && m; j++) {
-        const unsigned b = m & (0u - m);
-        keep |= b;
-        m ^= b;
-    }
-    return keep;
-}
-// A candidate the prefilter leaves undecided needs the reference distance on
-// its float position, a global load.  The first such candidate of a lane is
-// appended as inside and recorded in pend (row position << 12 | staged index);
-// after the scan the lane decides it, with one load round trip for the whole
-// wave, and turns it into the atom's own entry (which every consumer skips) if
-// it lies outside.  Further undecided candidates of the lane are decided at
-// once.  Candidates are staged indices q0 + k (k < n, n >= 1) with coarse
-// positions jp[k] = (x | y << 16, z); x holds the bits of the candidates to
-// leave out (the atom itself and its bonded partners; bits from kBuildChunk
-// up are ignored), bw = chi - clo is the width of the undecided band, slot_of
-// maps a staged index to its slot, and used[q] marks atom q as in a row.
-template <bool W16, class SlotOf>
-__device__ __forceinline__ void build_chunk_q(const uint2 (&jp)[kBuildChunk], unsigned pxy, unsigned pz, int clo,
-                                              unsigned bw, const FMD_GLOBAL float4* gpos, int q0, int n, float4 pi,
-                                              float L, float invL, float rcs2, unsigned x, FMD_GLOBAL int* out,
-                                              FMD_GLOBAL unsigned short* out16, int kcap, int& cnt, unsigned char* used,
-                                              int& pend, SlotOf slot_of) {
-    // t = q - clo is negative for a candidate certainly inside.  Its sign bit
-    // is shifted into m from the last candidate down (alignbit of (m, t) by 31
-    // is m << 1 | t >> 31), so bit k of m is candidate k; the smallest t as an
-    // unsigned number is the nearest candidate not certainly inside, and only
-    // when it lies in the band [0, bw] are the band's candidates found one by
-    // one.
-    unsigned m = 0u, umin = ~0u;
-    int t[kBuildChunk];
-#pragma unroll
-    for (int k = kBuildChunk - 1; k >= 0; k--) {
-        t[k] = coarse_t(pxy, pz, jp[k].x, jp[k].y, -clo);
-        m = __builtin_amdgcn_alignbit(m, (unsigned)t[k], 31);
-        umin = min(umin, (unsigned)t[k]);
-    }
-    const unsigned valid = (1u << min(n, kBuildChunk)) - 1u;  // k < n
-    m &= valid & ~x;
-    if (umin <= bw) {
-        unsigned band = 0u;
-#pragma unroll
-        for (int k = 0; k < kBuildChunk; k++) band |= ((unsigned)t[k] <= bw) ? (1u << k) : 0u;
-        band &= valid & ~x;
-        if (band && pend < 0) {  // defer the first: inside for now, its row position recorded
-            const int k = __builtin_ctz(band);
-            band &= band - 1u;
-            pend = ((cnt + __popc(m & ((1u << k) - 1u))) << 12) | (q0 + k);
-            m |= 1u << k;
-        }
-        for (int k = 0; k < kBuildChunk; k++)
-            if ((band >> k) & 1u)
-                m |= (dist2_ref(pi, gpos[slot_of(q0 + k)], L, invL) < rcs2) ? (1u << k) : 0u;
-    }
-    // the set bits in order, one pass per bit (a wave runs as many passes as
-    // its fullest lane has pairs in the chunk); entries past the row capacity
-    // are counted, not stored
-    const int p = __popc(m);
-    if (cnt + p > kcap) m = lowest_bits(m, kcap - cnt);
-    unsigned off = (unsigned)cnt * kTile;
-    cnt += p;
-    while (m) {
-        const int k = __builtin_ctz(m);
-        m &= m - 1u;
-        if (W16) out16[off] = (unsigned short)(q0 + k);
-        else out[off] = q0 + k;
-        used[q0 + k] = 1;
-        off += kTile;
-    }
-}
+// Rows are scanned in words of kWord candidates: a lane's hits among one word
+// are a 32-bit mask, kept with the word's first staged index until the rows
+// are placed.  At most kMaskWords words a tile, at the end of the tile's row
+// area (kMaskBytes; kMaskRows rows of 32-bit entries): far more than the
+// 9 rows x 2 words of a melt need, and a group with more takes the
+// global-memory scan.
+constexpr int kWord = 32;
+constexpr int kMaskWords = 64;
+constexpr int kMaskBytes = kMaskWords * kTile * 6;
+constexpr int kMaskRows = kMaskBytes / (kTile * 4);
+constexpr int kColWords = 18;  // words a row in the placement by columns
 
-// Block-wide exclusive prefix of one int per thread (kGroupSlots threads).
-__device__ inline int block_excl_scan(int x, int* s_wsum, int* total) {
-    const int lane = lane_id(), wv = threadIdx.x >> 6;
-    int v = x;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(v, o, 64);
-        if (lane >= o) v += y;
-    }
-    if (lane == 63) s_wsum[wv] = v;
-    __syncthreads();
-    int before = 0, all = 0;
-#pragma unroll
-    for (int w = 0; w < kGroupTiles; w++) {
-        const int ws = s_wsum[w];
-        before += (w < wv) ? ws : 0;
-        all += ws;
-    }
-    __syncthreads();
-    *total = all;
-    return before + v - x;
-}
-
-// At most 128 VGPRs (four waves per SIMD, four workgroups per CU with the
-// LDS below): the rebuilding replicas' groups fit in fewer rounds.
-__global__ void __launch_bounds__(kGroupSlots) __attribute__((amdgpu_waves_per_eu(4, 8))) k_build(REBUILD_ARGS) {
-    // staged union, coarse fixed point: x | y << 16 and z of each atom side by
-    // side (one chunk of padding: a cell's last chunk reads whole)
-    __shared__ uint2 s_pj[kBuildStage + kBuildChunk];
-    __shared__ unsigned short s_seg[kBuildStage];  // staged atom -> union cell
-    __shared__ unsigned char s_used[kBuildStage];  // staged atom is in a row of the group
-    __shared__ int4 s_cell[kMaxUnion];             // (first slot, count, LDS offset, key)
-    __shared__ unsigned int s_bits[kMaxWin / 32];   // union cells of the window
-    __shared__ unsigned char s_wmap[kMaxWin];       // window cell -> union index
-    __shared__ int s_red[6][kGroupTiles];           // per-wave window bounds
-    __shared__ int s_wsum[kGroupTiles];
-    __shared__ int s_c0[3], s_nu, s_nstage;
-    __shared__ int s_len[kGroupSlots];              // padded row length of each atom of the group
-    unsigned short* s_cidx = (unsigned short*)s_pj;  // after the scan: compact index of a used atom
+// The list build of one group by kGroupTiles x SPLIT waves.  Phases: the
+// union of the group's neighbor cells and its staging, the bonded tables, the
+// scan (hit masks), the neighbor set and the row lengths, the placement of the
+// rows from the masks.  Wave w works on tile w % kGroupTiles; with SPLIT > 1
+// each tile's nine rows of cells are shared out over its SPLIT waves (part
+// w / kGroupTiles), which keeps the order of the entries.
+//
+// What bounds it: instruction issue with every CU holding four groups (of a
+// group's 119 us in a 1M-bead melt the scan takes 37, the placement 28, the
+// bonded tables 11, the window and union 20), and one group's latency when
+// fewer groups than CUs are built (52 us).  Masks instead of appending each hit
+// as it is found: the rows are written once, whole 128-byte rows at a time
+// (appended, each lane's 2-byte stores fell in a row of their own, and the
+// rows were then read back and moved: 165 us a group), and the parts of a
+// split scan need not know their first entry.  Together per step: 1M beads
+// 230 -> 206 us, 128 uneven replicas 411 -> 364, 30,000 beads 49.0 -> 44.3.
+//
+// At most 128 VGPRs (four waves per SIMD: four workgroups of one wave per
+// tile, or one of four, per CU with the LDS below).
+template <int SPLIT>
+__global__ void __launch_bounds__(kGroupSlots * SPLIT) __attribute__((amdgpu_waves_per_eu(4, 8)))
+k_build(REBUILD_ARGS) {
+    constexpr int NT = kGroupSlots * SPLIT;
+    constexpr int WP = kMaskWords / SPLIT;  // words of one part
+    // During the scan s_raw holds
+    //   s_pj    staged union, coarse fixed point: x | y << 16 and z of each atom side
+    //           by side (one chunk of padding: a range's last chunk reads whole)
+    //   s_cell  union cells: (first slot, count, LDS offset, -)
+    //   s_seg   staged atom -> union cell
+    //   s_wmap  window cell -> union index
+    // and for the placement of a group whose neighbor set fits
+    //   s_cidx  LDS byte offset of a used atom
+    //   s_m, s_q  the hit masks and their first staged indices, by column
+    constexpr int kPj = (kBuildStage + kBuildChunk) * 8, kCell = kMaxUnion * 16, kSeg = kBuildStage * 2;
+    constexpr int kCidx = kBuildStage * 2, kMs = kColWords * kGroupSlots * 4, kQs = kColWords * kGroupSlots * 2;
+    static_assert(kCidx + kMs + kQs <= kPj + kCell + kSeg + kMaxWin, "the masks fit the scan's arrays");
+    __shared__ __align__(16) char s_raw[kPj + kCell + kSeg + kMaxWin];
+    uint2* const s_pj = (uint2*)s_raw;
+    int4* const s_cell = (int4*)(s_raw + kPj);
+    unsigned short* const s_seg = (unsigned short*)(s_raw + kPj + kCell);
+    unsigned char* const s_wmap = (unsigned char*)(s_raw + kPj + kCell + kSeg);
+    unsigned short* const s_cidx = (unsigned short*)s_raw;
+    unsigned* const s_m = (unsigned*)(s_raw + kCidx);
+    unsigned short* const s_q = (unsigned short*)(s_raw + kCidx + kMs);
+    __shared__ uint2 s_used[kBuildStage / 32 + 1];  // staged atoms in a row of the group: bits, set bits before
+    __shared__ unsigned int s_bits[kMaxWin / 32];  // union cells of the window
+    __shared__ int s_wpre[kMaxWin / 32];           // union cells before each word of the window
+    __shared__ int s_red[6][kGroupTiles];          // per-wave window bounds
+    __shared__ int s_c0[3], s_nu, s_nstage, s_ncomp, s_flag;
+    __shared__ int s_cnt[SPLIT][kGroupSlots];      // hits of each atom, by part
+    __shared__ unsigned char s_words[SPLIT][kGroupSlots];  // and words
+    __shared__ unsigned s_col[kGroupSlots];        // by column: row entries | padding entry << 16
+    __shared__ int s_hist[kGroupTiles][64];        // rows of each padded length (in kLJTail), by tile
+    __shared__ int s_tlen[kGroupTiles];
+    __shared__ unsigned short s_rank[kGroupSlots];  // column of each atom's row
+    // s_flag: a partner outside the set; too many words or hits; too many words for the column form
+    constexpr int kMiss = 1, kOver = 2, kMany = 4;
     // the wave index as a scalar: each wave's tile and replica fields are uniform
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_id(), tid = threadIdx.x;
+    const int tl = wv % kGroupTiles, part = wv / kGroupTiles, at = tl * kTile + lane;
     for (int gb = blockIdx.x, ng = *nrt / kGroupTiles; gb < ng; gb += gridDim.x) {
-        const Tile t = tiles[rlist[gb * kGroupTiles + wv]];
+        const Tile t = tiles[rlist[gb * kGroupTiles + tl]];
         const RepDesc& d = descs[t.rep];
         RepState* st = d.st;
         const int i = t.lt * kTile + lane;
         const int grp = t.lt / kGroupTiles;
         const bool valid = i < d.natoms;
         int err = 0;
-        // bonded partners (slots), the exclusion set and the bonded tables
-        int ex[4] = {-1, -1, -1, -1};
+        // the exclusion set: the first four bonded partners (slots), and their
+        // entries in the topology
+        int ex[4] = {-1, -1, -1, -1}, ent[4] = {0, 0, 0, 0};
         int nb = 0;
         float4 pi = make_float4(0.f, 0.f, 0.f, 0.f);
+        int4 pf = make_int4(0, 0, 0, 0);
         if (valid) {
             pi = gview(d.pos)[i];
-            const int g = gview(d.img)[i].w;
-            const int b0 = gview(d.t_boff)[g], b1 = gview(d.t_boff)[g + 1];
-            for (int e = b0; e < b1; e++) {
-                const int ent = gview(d.t_blst)[e];
-                const int ps = gview(d.slot_of)[ent & kSlotMask];
-                if (nb < d.bcap) gmut(d.bnd)[((size_t)t.lt * d.bcap + nb) * kTile + lane] = ps | (ent & ~kSlotMask);
-                if (nb < 4) ex[nb] = ps;
-                nb++;
-            }
-            if (nb > d.bcap) err |= ERR_BONDED;
-            int na = 0;
-            const int a0 = gview(d.t_aoff)[g], a1 = gview(d.t_aoff)[g + 1];
-            for (int e = a0; e < a1; e++) {
-                const int4 A = gview(d.t_alst)[e];
-                const int role = (A.x == g) ? 0 : ((A.y == g) ? 1 : 2);
-                const int o1 = (role == 0) ? A.y : A.x;
-                const int o2 = (role == 2) ? A.y : A.z;
-                const int s1 = gview(d.slot_of)[o1], s2 = gview(d.slot_of)[o2];
-                if (na < d.acap)
-                    gmut(d.ang)[((size_t)t.lt * d.acap + na) * kTile + lane] =
-                        make_int2(s1 | (role << kSlotBits), s2 | (A.w << kSlotBits));
-                na++;
-            }
-            if (na > d.acap) err |= ERR_BONDED;
-            gmut(d.bhdr)[i] = min(nb, d.bcap) | (min(na, d.acap) << 8);
+            pf = (int4)gview(d.ipos)[i];
+            const int gid = gview(d.gid)[i], b0 = gview(d.t_boff)[gid];
+            nb = gview(d.t_boff)[gid + 1] - b0;
+#pragma unroll
+            for (int b = 0; b < 4; b++)
+                if (b < nb) ent[b] = gview(d.t_blst)[b0 + b];
+#pragma unroll
+            for (int b = 0; b < 4; b++)
+                if (b < nb) ex[b] = gview(d.slot_of)[ent[b] & kSlotMask];
         }
-        const FMD_GLOBAL int* bt = gview(d.bnd) + (size_t)t.lt * d.bcap * kTile + lane;
-        FMD_GLOBAL int* out = gmut(d.nbr) + (size_t)t.lt * d.kcap * kTile + lane;
-        // 16-bit rows are built in the upper half of the tile's row area (which
-        // holds 2 kcap 16-bit entries per lane) and moved to the lower half by
-        // the placement below; 32-bit rows are built in place
-        FMD_GLOBAL unsigned short* out16 =
-            (FMD_GLOBAL unsigned short*)(gmut(d.nbr) + (size_t)t.lt * d.kcap * kTile) + (size_t)d.kcap * kTile + lane;
         const int kcap = d.kcap;
         const float rcs2 = d.rcs2;
-        const int nx = st->nx;
-        const float ics = st->inv_cs;
-        const float L = st->Lp, invL = st->invLp;
+        auto uni = [](float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); };
+        const int nx = __builtin_amdgcn_readfirstlane(st->nx);
+        const float ics = uni(st->inv_cs);
+        const float L = uni(st->Lp), invL = uni(st->invLp);
         const FMD_GLOBAL float4* gpos = gview(d.pos);
         const FMD_GLOBAL int* cstart = gview(d.cell_start);
         int cx = 0, cy = 0, cz = 0;
@@ -1006,7 +928,11 @@ __global__ void __launch_bounds__(kGroupSlots) __attribute__((amdgpu_waves_per_e
         // by one cell per side (the whole axis if that wraps): a window of at
         // most kMaxWin cells.  A bitmap over the window marks the union, whose
         // cells are numbered in window order.
-        if (tid == 0) { s_c0[0] = cx; s_c0[1] = cy; s_c0[2] = cz; }
+        if (tid == 0) { s_c0[0] = cx; s_c0[1] = cy; s_c0[2] = cz; s_flag = 0; }
+        for (int j = tid; j < kMaxWin / 32; j += NT) s_bits[j] = 0u;
+        for (int j = tid; j < kBuildStage / 32 + 1; j += NT) s_used[j].x = 0u;
+        if (tid < kGroupTiles * 64) s_hist[tid / 64][tid % 64] = 0;
+        if (tid < kGroupTiles) s_tlen[tid] = 0;
         __syncthreads();
         const int h = nx >> 1;
         auto rel = [&](int c, int c0) {
@@ -1015,15 +941,16 @@ __global__ void __launch_bounds__(kGroupSlots) __attribute__((amdgpu_waves_per_e
             r -= (r >= nx - h) ? nx : 0;
             return r;
         };
-        const int c0x = s_c0[0], c0y = s_c0[1], c0z = s_c0[2];
+        const int c0x = __builtin_amdgcn_readfirstlane(s_c0[0]), c0y = __builtin_amdgcn_readfirstlane(s_c0[1]),
+                  c0z = __builtin_amdgcn_readfirstlane(s_c0[2]);
         const int rx = valid ? rel(cx, c0x) : 0, ry = valid ? rel(cy, c0y) : 0, rz = valid ? rel(cz, c0z) : 0;
-        {
+        if (part == 0) {
             const int lo_x = wave_min_i(valid ? rx : INT_MAX), hi_x = wave_max_i(valid ? rx : INT_MIN);
             const int lo_y = wave_min_i(valid ? ry : INT_MAX), hi_y = wave_max_i(valid ? ry : INT_MIN);
             const int lo_z = wave_min_i(valid ? rz : INT_MAX), hi_z = wave_max_i(valid ? rz : INT_MIN);
             if (lane == 0) {
-                s_red[0][wv] = lo_x; s_red[1][wv] = hi_x; s_red[2][wv] = lo_y;
-                s_red[3][wv] = hi_y; s_red[4][wv] = lo_z; s_red[5][wv] = hi_z;
+                s_red[0][tl] = lo_x; s_red[1][tl] = hi_x; s_red[2][tl] = lo_y;
+                s_red[3][tl] = hi_y; s_red[4][tl] = lo_z; s_red[5][tl] = hi_z;
             }
         }
         __syncthreads();
@@ -1031,47 +958,27 @@ __global__ void __launch_bounds__(kGroupSlots) __attribute__((amdgpu_waves_per_e
         auto window = [&](int a, int& s0, int& e0) {
             int lo = INT_MAX, hi = INT_MIN;
             for (int w = 0; w < kGroupTiles; w++) { lo = min(lo, s_red[2 * a][w]); hi = max(hi, s_red[2 * a + 1][w]); }
-            s0 = lo - 1;
-            e0 = min(hi - lo + 3, nx);  // the whole axis once the grown box wraps
+            s0 = __builtin_amdgcn_readfirstlane(lo - 1);
+            e0 = __builtin_amdgcn_readfirstlane(min(hi - lo + 3, nx));  // the whole axis once the grown box wraps
         };
         window(0, sx, ex_);
         window(1, sy, ey_);
         window(2, sz, ez_);
-        // window cell of this atom's neighbor cell c in (dz, dy, dx) order; the
-        // offset from the window start is >= 0 and, on an axis the window
-        // wraps (extent nx), taken modulo nx
+        // window cell of this atom's neighbor cell (dx, dy, dz); the offset from
+        // the window start is >= 0 and, on an axis the window wraps (extent nx),
+        // taken modulo nx
         auto wmod = [](int v, int e) {  // v in [0, e + 1]: v mod e (e >= 1)
             v -= (v >= e) ? e : 0;
             v -= (v >= e) ? e : 0;
             return v;
         };
-        auto win_of = [&](int c) {
-            const int wx = wmod(rx + c % 3 - 1 - sx, ex_), wy = wmod(ry + (c / 3) % 3 - 1 - sy, ey_),
-                      wz = wmod(rz + c / 9 - 1 - sz, ez_);
-            return (wz * ey_ + wy) * ex_ + wx;
+        auto win_at = [&](int dx, int dy, int dz) {
+            return (wmod(rz + dz - sz, ez_) * ey_ + wmod(ry + dy - sy, ey_)) * ex_ + wmod(rx + dx - sx, ex_);
         };
         const int W = ex_ * ey_ * ez_;
-        // The staged index of a bonded partner (slot ps): its cell is one of the
-        // 27 around this atom's (a bond is shorter than a cell), found through
-        // the window; -1 if not (the group then keeps slots everywhere).
-        auto partner_q = [&](int ps) __attribute__((always_inline)) -> int {
-            const float4 pp = gpos[ps];
-            int dx = cell_coord(pp.x, ics, nx) - cx, dy = cell_coord(pp.y, ics, nx) - cy,
-                dz = cell_coord(pp.z, ics, nx) - cz;
-            dx += (dx < -1) ? nx : 0; dx -= (dx > 1) ? nx : 0;
-            dy += (dy < -1) ? nx : 0; dy -= (dy > 1) ? nx : 0;
-            dz += (dz < -1) ? nx : 0; dz -= (dz > 1) ? nx : 0;
-            if (dx < -1 || dx > 1 || dy < -1 || dy > 1 || dz < -1 || dz > 1) return -1;
-            const int u = s_wmap[win_of((dz + 1) * 9 + (dy + 1) * 3 + (dx + 1))];
-            if (u >= s_nu) return -1;
-            const int4 ce = s_cell[u];
-            const int o = ps - ce.x;
-            return (o >= 0 && o < ce.y) ? ce.z + o : -1;
-        };
         // staged scan: prefilter in fixed point; boxes of fewer than 3 cells per
         // axis (where a pair can sit near half the box) use the global scan
         bool staged = W <= kMaxWin && nx >= 3;  // uniform over the group
-        const int4 pf = valid ? (int4)gview(d.ipos)[i] : make_int4(0, 0, 0, 0);
         const unsigned cxy = coarse_xy(pf), cz16 = coarse_z(pf);
         int clo, chi, rb2;
         {
@@ -1081,412 +988,702 @@ __global__ void __launch_bounds__(kGroupSlots) __attribute__((amdgpu_waves_per_e
             const double band = 3e-5 + 1e-6 * (double)L / (double)d.rcs;  // >> the two forms' difference
             const double rb = rc * sqrt(1.0 + band);  // above the true distance of any pair the FP32 test accepts
             const double rin = rc * sqrt(1.0 - band) - 1.7321 - 0.01, rout = rb + 1.7321 + 0.01;
-            clo = rin > 0.0 ? (int)floor(rin * rin) : 0;
-            chi = (int)ceil(rout * rout);
-            rb2 = (int)fmin(ceil(rb * rb) + 1.0, 2147483647.0);
+            clo = __builtin_amdgcn_readfirstlane(rin > 0.0 ? (int)floor(rin * rin) : 0);
+            chi = __builtin_amdgcn_readfirstlane((int)ceil(rout * rout));
+            rb2 = __builtin_amdgcn_readfirstlane((int)fmin(ceil(rb * rb) + 1.0, 2147483647.0));
         }
         int nu = 0, nstage = 0;
         if (staged) {
-            for (int j = tid; j < kMaxWin / 32; j += kGroupSlots) s_bits[j] = 0u;
-            __syncthreads();
-            // each cell of the group marks its 27 neighbors (its first lane in a wave does)
+            // each cell of the group marks its 27 neighbors (its first lane in a
+            // wave does), a share of them in each part
             const int prev = __shfl_up(cx + nx * (cy + nx * cz), 1, 64);
             if (valid && (lane == 0 || prev != cx + nx * (cy + nx * cz)))
                 #pragma unroll 1
-                for (int c = 0; c < 27; c++) {
-                    const int w = win_of(c);
+                for (int c = part; c < 27; c += SPLIT) {
+                    const int w = win_at(c % 3 - 1, (c / 3) % 3 - 1, c / 9 - 1);
                     atomicOr(&s_bits[w >> 5], 1u << (w & 31));
                 }
             __syncthreads();
             if (wv == 0) {
-                // number the marked cells in window order
+                // marked cells before each word of the window
                 const int nwords = (W + 31) >> 5;  // <= kMaxWin / 32 <= 64 lanes
-                const unsigned bits = (lane < nwords) ? s_bits[lane] : 0u;
-                int x = __popc(bits);
+                const int c = (lane < nwords) ? __popc(s_bits[lane]) : 0;
+                int x = c;
 #pragma unroll
                 for (int o = 1; o < 64; o <<= 1) {
                     const int y = __shfl_up(x, o, 64);
                     if (lane >= o) x += y;
                 }
-                const int nuw = __shfl(x, 63, 64);
-                if (lane == 0) s_nu = nuw;
-                if (nuw <= kMaxUnion) {
-                    // lane l numbers bit (l & 31) of word j + (l >> 5): two words per pass
-                    const int base = x - __popc(bits);  // marked cells in words below this lane's word
-                    auto wrapn = [&](int p) {           // p in [-nx, 2 nx)
-                        p += (p < 0) ? nx : 0;
-                        p -= (p >= nx) ? nx : 0;
-                        return p;
-                    };
-                    for (int j = 0; j < nwords; j += 2) {
-                        const int word = j + (lane >> 5), bit = lane & 31;
-                        const unsigned wb = __shfl(bits, word & 63, 64);
-                        const int wbase = __shfl(base, word & 63, 64);
-                        if (word < nwords && ((wb >> bit) & 1u)) {
-                            const int w = word * 32 + bit;
-                            const int u = wbase + __popc(wb & ((1u << bit) - 1u));
-                            const int wx = w % ex_, wy = (w / ex_) % ey_, wz = w / (ex_ * ey_);
-                            s_wmap[w] = (unsigned char)u;
-                            s_cell[u] = make_int4(0, 0, 0, (int)cell_key(wrapn(c0x + sx + wx),
-                                                                         wrapn(c0y + sy + wy),
-                                                                         wrapn(c0z + sz + wz)));
-                        }
-                    }
-                    // counts and LDS offsets of the union cells
-                    int ns = 0;
-                    for (int u0 = 0; u0 < nuw; u0 += 64) {
-                        const int u = u0 + lane;
-                        int s0 = 0, c = 0;
-                        if (u < nuw) {
-                            const int k = s_cell[u].w;
-                            s0 = cstart[k];
-                            c = cstart[k + 1] - s0;
-                        }
-                        int y = c;
-#pragma unroll
-                        for (int o = 1; o < 64; o <<= 1) {
-                            const int z = __shfl_up(y, o, 64);
-                            if (lane >= o) y += z;
-                        }
-                        if (u < nuw) s_cell[u] = make_int4(s0, c, ns + y - c, s_cell[u].w);
-                        ns += __shfl(y, 63, 64);
-                    }
-                    if (lane == 0) s_nstage = ns;
+                if (lane < nwords) s_wpre[lane] = x - c;
+                if (lane == 63) s_nu = x;
+            }
+            __syncthreads();
+            nu = __builtin_amdgcn_readfirstlane(s_nu);
+            staged = nu <= kMaxUnion;
+        }
+        if (staged) {
+            // number the marked cells in window order, with their slots
+            auto wrapn = [&](int p) {  // p in [-nx, 2 nx)
+                p += (p < 0) ? nx : 0;
+                p -= (p >= nx) ? nx : 0;
+                return p;
+            };
+            for (int w = tid; w < W; w += NT) {
+                const unsigned wb = s_bits[w >> 5];
+                if ((wb >> (w & 31)) & 1u) {
+                    const int u = s_wpre[w >> 5] + __popc(wb & ((1u << (w & 31)) - 1u));
+                    const int wx = w % ex_, wyz = w / ex_, wy = wyz % ey_, wz = wyz / ey_;
+                    const int k = (int)cell_key(wrapn(c0x + sx + wx), wrapn(c0y + sy + wy), wrapn(c0z + sz + wz));
+                    const int s0 = cstart[k];
+                    s_wmap[w] = (unsigned char)u;
+                    s_cell[u] = make_int4(s0, cstart[k + 1] - s0, 0, 0);
                 }
             }
             __syncthreads();
-            nu = s_nu;
-            staged = nu <= kMaxUnion;
-            if (staged) {
-                nstage = s_nstage;
-                staged = nstage <= kBuildStage;
+            if (wv == 0) {  // LDS offsets of the union cells
+                int ns = 0;
+                for (int u0 = 0; u0 < nu; u0 += 64) {
+                    const int u = u0 + lane;
+                    const int c = (u < nu) ? s_cell[u].y : 0;
+                    int y = c;
+#pragma unroll
+                    for (int o = 1; o < 64; o <<= 1) {
+                        const int z = __shfl_up(y, o, 64);
+                        if (lane >= o) y += z;
+                    }
+                    if (u < nu) s_cell[u].z = ns + y - c;
+                    ns += __shfl(y, 63, 64);
+                }
+                if (lane == 0) s_nstage = ns;
             }
+            __syncthreads();
+            nstage = __builtin_amdgcn_readfirstlane(s_nstage);
+            staged = nstage <= kBuildStage;
         }
         if (staged) {
-            for (int u = tid; u < nu; u += kGroupSlots) {
+            for (int u = tid; u < nu; u += NT) {
                 const int4 ce = s_cell[u];
                 for (int j = 0; j < ce.y; j++) s_seg[ce.z + j] = (unsigned short)u;
             }
-            for (int q = tid; q < nstage; q += kGroupSlots) s_used[q] = 0;
             __syncthreads();
             const FMD_GLOBAL int4* gip = gview(d.ipos);
-            for (int q0 = 0; q0 < nstage; q0 += 4 * kGroupSlots) {
-                int4 v4[4];
+            constexpr int kAhead = SPLIT == 1 ? 4 : 2;  // positions in flight per thread
+            for (int q0 = 0; q0 < nstage; q0 += kAhead * NT) {
+                int4 v4[kAhead];
 #pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const int q = min(q0 + k * kGroupSlots + tid, nstage - 1);
+                for (int k = 0; k < kAhead; k++) {
+                    const int q = min(q0 + k * NT + tid, nstage - 1);
                     const int4 ce = s_cell[s_seg[q]];
                     v4[k] = gip[ce.x + q - ce.z];
                 }
 #pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const int q = q0 + k * kGroupSlots + tid;
+                for (int k = 0; k < kAhead; k++) {
+                    const int q = q0 + k * NT + tid;
                     if (q < nstage) s_pj[q] = make_uint2(coarse_xy(v4[k]), coarse_z(v4[k]));
                 }
             }
             __syncthreads();
         }
-        int cnt = 0, qself = 0, pend = -1;
-        if (valid && staged) {
-            {  // the atom's own staged index (its own cell is window cell win_of(13))
-                const int us = s_wmap[win_of(13)];
-                if (us < nu) qself = s_cell[us].z + (i - s_cell[us].x);
-            }
-            // exclusions as staged indices: the atom itself and its first four
-            // bonded partners (none, or a partner outside the 27 cells, which is
-            // no candidate: INT_MAX)
-            int xs[5] = {qself, INT_MAX, INT_MAX, INT_MAX, INT_MAX};
+        auto slot_of = [&](int q) __attribute__((always_inline)) {  // slot of a staged atom
+            const int4 ce = s_cell[s_seg[q]];
+            return ce.x + q - ce.z;
+        };
+        auto mark = [&](int q) __attribute__((always_inline)) { atomicOr(&s_used[q >> 5].x, 1u << (q & 31)); };
+        // The staged index of a bonded partner (slot ps at position pp): its cell
+        // is one of the 27 around this atom's (a bond is shorter than a cell),
+        // found through the window; -1 if not (the group then keeps slots
+        // everywhere).
+        auto staged_of = [&](int ps, float4 pp) __attribute__((always_inline)) -> int {
+            int dx = rel(cell_coord(pp.x, ics, nx), c0x) - rx, dy = rel(cell_coord(pp.y, ics, nx), c0y) - ry,
+                dz = rel(cell_coord(pp.z, ics, nx), c0z) - rz;
+            dx += (dx < -1) ? nx : 0; dx -= (dx > 1) ? nx : 0;
+            dy += (dy < -1) ? nx : 0; dy -= (dy > 1) ? nx : 0;
+            dz += (dz < -1) ? nx : 0; dz -= (dz > 1) ? nx : 0;
+            if (dx < -1 || dx > 1 || dy < -1 || dy > 1 || dz < -1 || dz > 1) return -1;
+            const int u = s_wmap[win_at(dx, dy, dz)];
+            if (u >= nu) return -1;
+            const int4 ce = s_cell[u];
+            const int o = ps - ce.x;
+            return (o >= 0 && o < ce.y) ? ce.z + o : -1;
+        };
+        // exclusions as staged indices: the first four bonded partners (none, or a
+        // partner outside the 27 cells, which is no candidate: INT_MAX).  Their
+        // positions are requested together, so the latencies overlap.
+        int xs[4] = {INT_MAX, INT_MAX, INT_MAX, INT_MAX};
+        if (staged && valid) {
+            float4 pp[4];
+#pragma unroll
+            for (int b = 0; b < 4; b++) pp[b] = gpos[ex[b] >= 0 ? ex[b] : i];
 #pragma unroll
             for (int b = 0; b < 4; b++) {
-                const int q = ex[b] >= 0 ? partner_q(ex[b]) : -1;
-                xs[b + 1] = q >= 0 ? q : INT_MAX;
+                const int q = ex[b] >= 0 ? staged_of(ex[b], pp[b]) : -1;
+                xs[b] = q >= 0 ? q : INT_MAX;
             }
-            int nxu = 1;  // entries from nxu on are INT_MAX in every lane of the wave
+        }
+        // The bonded tables, the bonds by part 0 and the angles by the last:
+        // entries hold the partners' slots, or with `set` their staged indices
+        // (marked as used), which become LDS byte offsets once the set is known.
+        const bool do_bonds = part == 0, do_angles = part == SPLIT - 1;
+        int miss = 0;
+        auto use = [&](int q) __attribute__((always_inline)) {  // a partner's staged index as an entry
+            const bool in = q >= 0 && q != INT_MAX;
+            if (in) mark(q);
+            else miss = 1;
+            return in ? q : 0;
+        };
+        auto partner = [&](int b) __attribute__((always_inline)) {  // the slot of bonded partner b >= 4
+            return (int)gview(d.slot_of)[gview(d.t_blst)[gview(d.t_boff)[gview(d.gid)[i]] + b] & kSlotMask];
+        };
+        auto bonded = [&](bool set) __attribute__((always_inline)) {
+            const int gid = gview(d.gid)[i], a0 = gview(d.t_aoff)[gid], na = gview(d.t_aoff)[gid + 1] - a0;
+            if (do_bonds) {
+                FMD_GLOBAL int* bt = gmut(d.bnd) + (size_t)t.lt * d.bcap * kTile + lane;
+                const int nbk = min(nb, d.bcap);
+                gmut(d.bhdr)[i] = nbk | (min(na, d.acap) << 8);
+                if (nb > d.bcap || na > d.acap) err |= ERR_BONDED;
 #pragma unroll
-            for (int b = 1; b < 5; b++) nxu = __ballot(xs[b] != INT_MAX) ? b + 1 : nxu;
-            auto slot_of = [&](int q) __attribute__((always_inline)) {
-                const int4 ce = s_cell[s_seg[q]];
-                return ce.x + q - ce.z;
-            };
-            // Lower bounds (coarse units) of the distance along y and z from
-            // this atom to any atom of the cell below and above its own: its
-            // offset from its cell's bounds floor(c 2^16 / nx), less 2 units
-            // (the truncation of the atom's coordinate and of the bound, and
-            // the rounding of the float cell coordinate).  With 5 or more cells
-            // per axis these offsets, taken as signed 16-bit differences, do
-            // not wrap.
-            int yb[2] = {0, 0}, zb[2] = {0, 0};
-            const bool trim = nx >= 5;
-            if (trim) {
-                auto cb = [&](int c) { return (int)(((unsigned)c << 16) / (unsigned)nx); };
-                auto off16 = [](int a, int b) { return max(0, (int)(short)(unsigned short)(a - b) - 2); };
-                const int yc = (int)(cxy >> 16), zc = (int)cz16;
-                yb[0] = off16(yc, cb(cy)); yb[1] = off16(cb(cy + 1), yc);
-                zb[0] = off16(zc, cb(cz)); zb[1] = off16(cb(cz + 1), zc);
-            }
-            // x offset of staged atom q from this atom (coarse units, signed)
-            auto dxc = [&](int q) { return (int)(short)(unsigned short)(s_pj[q].x - cxy); };
-            // first q in [lo, hi) with dxc(q) > v: a cell's atoms are in
-            // ascending x, and so are the three cells of a row in x order
-            auto first_above = [&](int lo, int hi, int v) {
-                while (lo < hi) {
-                    const int mid = (lo + hi) >> 1;
-                    if (dxc(mid) <= v) lo = mid + 1;
-                    else hi = mid;
+                for (int b = 0; b < 4; b++)
+                    if (b < nbk) bt[b * kTile] = (set ? use(xs[b]) : ex[b]) | (ent[b] & ~kSlotMask);
+                for (int b = 4; b < nbk; b++) {
+                    const int ps = partner(b);
+                    bt[b * kTile] = (set ? use(staged_of(ps, gpos[ps])) : ps) |
+                                    (gview(d.t_blst)[gview(d.t_boff)[gid] + b] & ~kSlotMask);
                 }
-                return lo;
-            };
-            auto scan_rows = [&](auto w16) __attribute__((always_inline)) {
-                constexpr bool W16 = decltype(w16)::value;
-                auto scan_range = [&](int z, int e) __attribute__((always_inline)) {
-                    for (int q0 = z; q0 < e; q0 += kBuildChunk) {
-                        // a whole chunk from LDS (entries past the range are
-                        // masked out, and the array is padded by a chunk)
+            }
+            if (do_angles) {
+                // kAngles at a time, the loads of each step of their chains together
+                constexpr int kAngles = 3;
+                FMD_GLOBAL int2* an = gmut(d.ang) + (size_t)t.lt * d.acap * kTile + lane;
+                const int nak = min(na, d.acap);
+                for (int k0 = 0; k0 < nak; k0 += kAngles) {
+                    int4 A[kAngles];
+                    int s1[kAngles], s2[kAngles], role[kAngles];
+#pragma unroll
+                    for (int k = 0; k < kAngles; k++) A[k] = (int4)gview(d.t_alst)[a0 + min(k0 + k, nak - 1)];
+#pragma unroll
+                    for (int k = 0; k < kAngles; k++) {
+                        role[k] = (A[k].x == gid) ? 0 : ((A[k].y == gid) ? 1 : 2);
+                        s1[k] = gview(d.slot_of)[role[k] == 0 ? A[k].y : A[k].x];
+                        s2[k] = gview(d.slot_of)[role[k] == 2 ? A[k].y : A[k].z];
+                    }
+                    float4 p1[kAngles], p2[kAngles];
+                    if (set) {
+#pragma unroll
+                        for (int k = 0; k < kAngles; k++) { p1[k] = gpos[s1[k]]; p2[k] = gpos[s2[k]]; }
+                    }
+#pragma unroll
+                    for (int k = 0; k < kAngles; k++)
+                        if (k0 + k < nak) {
+                            const int e1 = set ? use(staged_of(s1[k], p1[k])) : s1[k];
+                            const int e2 = set ? use(staged_of(s2[k], p2[k])) : s2[k];
+                            an[(k0 + k) * kTile] = make_int2(e1 | (role[k] << kSlotBits), e2 | (A[k].w << kSlotBits));
+                        }
+                }
+            }
+        };
+        const bool want_set = staged && !d.nostage;  // uniform
+        if (valid) bonded(want_set);
+        // hit masks of this lane and part, in row order
+        char* const area_end = (char*)(d.nbr + (size_t)(t.lt + 1) * d.kcap * kTile);
+        FMD_GLOBAL unsigned* gm = gmut((unsigned*)(area_end - kMaskBytes)) + part * WP * kTile + lane;
+        FMD_GLOBAL unsigned short* gq =
+            gmut((unsigned short*)(area_end - kMaskBytes + kMaskWords * kTile * 4)) + part * WP * kTile + lane;
+        int cnt = 0, qself = 0, nw = 0;
+        if (staged) {
+            int pend = -1, pq = 0, over = 0;
+            if (valid) {
+                {  // the atom's own staged index
+                    const int us = s_wmap[win_at(0, 0, 0)];
+                    if (us < nu) qself = s_cell[us].z + (i - s_cell[us].x);
+                    if (us >= nu || qself < 0 || qself >= nstage) {
+                        err |= ERR_INTERNAL;
+                        qself = 0;
+                    }
+                    if (part == 0) mark(qself);
+                }
+                int nxu = 0;  // entries of xs from nxu on are INT_MAX in every lane of the wave
+#pragma unroll
+                for (int b = 0; b < 4; b++) nxu = __ballot(xs[b] != INT_MAX) ? b + 1 : nxu;
+                // Lower bounds (coarse units) of the distance along y and z from
+                // this atom to any atom of the cell below and above its own: its
+                // offset from its cell's bounds floor(c 2^16 / nx), less 2 units
+                // (the truncation of the atom's coordinate and of the bound, and
+                // the rounding of the float cell coordinate).  These offsets are
+                // less than two cells, so with 3 or more cells per axis they do not
+                // wrap as signed 16-bit differences of at most one cell.
+                int yb[2], zb[2];
+                {
+                    auto cb = [&](int c) { return (int)(((unsigned)c << 16) / (unsigned)nx); };
+                    auto off16 = [](int a, int b) { return max(0, (int)(short)(unsigned short)(a - b) - 2); };
+                    const int yc = (int)(cxy >> 16), zc = (int)cz16;
+                    yb[0] = off16(yc, cb(cy)); yb[1] = off16(cb(cy + 1), yc);
+                    zb[0] = off16(zc, cb(cz)); zb[1] = off16(cb(cz + 1), zc);
+                }
+                // First q in [lo, hi) whose x offset from this atom, less `by`, is
+                // above v (coarse units).  A cell's atoms are in ascending x; their
+                // offsets from an atom of the neighboring cell span two cells, which
+                // may wrap as signed 16-bit numbers, but not those less one cell
+                // (by = -cell or cell, the offset of the cell's middle).
+                const int cell16 = (int)(65536u / (unsigned)nx);
+                auto first_above = [&](int lo, int hi, int by, int v) {
+                    const unsigned ref = (cxy & 0xFFFFu) + (unsigned)by;
+                    while (lo < hi) {
+                        const int mid = (lo + hi) >> 1;
+                        if ((int)(short)(unsigned short)(s_pj[mid].x - ref) <= v) lo = mid + 1;
+                        else hi = mid;
+                    }
+                    return lo;
+                };
+                const unsigned bw = (unsigned)(chi - clo);
+                // the hits among the candidates q0 .. q0 + n - 1 (n <= kWord): chunks
+                // of kBuildChunk by the coarse prefilter.  t = q - clo is negative for
+                // a candidate certainly inside; its sign bit is shifted into m from the
+                // last candidate down (alignbit of (m, t) by 31 is m << 1 | t >> 31),
+                // so bit k of m is candidate k; the smallest t as an unsigned number is
+                // the nearest candidate not certainly inside, and only when it lies in
+                // the band [0, bw] are the band's candidates found one by one.
+                auto word = [&](int q0, int n) __attribute__((always_inline)) {
+                    unsigned m = 0u, band = 0u;
+#pragma unroll
+                    for (int c = 0; c < kWord; c += kBuildChunk) {
+                        if (c >= n) break;
+                        unsigned m8 = 0u, umin = ~0u;
+                        int tt[kBuildChunk];
                         uint2 jp[kBuildChunk];
 #pragma unroll
-                        for (int k = 0; k < kBuildChunk; k++) jp[k] = s_pj[q0 + k];
-                        // bit xs[b] - q0 for each exclusion; one outside the
-                        // chunk lands on a bit from 8 to 31, which is dropped
-                        auto xbit = [&](int v) { return 1u << min((unsigned)(v - q0), 31u); };
-                        unsigned x = xbit(xs[0]) | xbit(xs[1]) | xbit(xs[2]);
-                        if (__builtin_expect(nxu > 3, 0)) x |= xbit(xs[3]) | xbit(xs[4]);
-                        for (int b = 4; b < nb && b < d.bcap; b++) {  // partners past the first four
-                            const unsigned o = (unsigned)(partner_q(bt[b * kTile] & kSlotMask) - q0);
-                            x |= (o < (unsigned)kBuildChunk) ? (1u << o) : 0u;
+                        for (int k = 0; k < kBuildChunk; k++) jp[k] = s_pj[q0 + c + k];
+#pragma unroll
+                        for (int k = kBuildChunk - 1; k >= 0; k--) {
+                            tt[k] = coarse_t(cxy, cz16, jp[k].x, jp[k].y, -clo);
+                            m8 = __builtin_amdgcn_alignbit(m8, (unsigned)tt[k], 31);
+                            umin = min(umin, (unsigned)tt[k]);
                         }
-                        build_chunk_q<W16>(jp, cxy, cz16, clo, (unsigned)(chi - clo), gpos, q0, e - q0, pi, L, invL,
-                                           rcs2, x, out, out16, kcap, cnt, s_used, pend, slot_of);
+                        m |= m8 << c;
+                        if (umin <= bw) {
+#pragma unroll
+                            for (int k = 0; k < kBuildChunk; k++) band |= ((unsigned)tt[k] <= bw) ? (1u << (c + k)) : 0u;
+                        }
+                    }
+                    unsigned keep = n >= kWord ? ~0u : (1u << n) - 1u;
+                    // leave out the atom itself and its bonded partners
+                    auto drop = [&](int v) {
+                        const unsigned o = (unsigned)(v - q0);
+                        keep &= ~(o < (unsigned)kWord ? 1u << o : 0u);
+                    };
+                    drop(qself); drop(xs[0]); drop(xs[1]);
+                    if (__builtin_expect(nxu > 2, 0)) { drop(xs[2]); drop(xs[3]); }
+                    for (int b = 4; b < nb; b++) {  // partners past the first four
+                        const int ps = partner(b), q = staged_of(ps, gpos[ps]);
+                        if (q >= 0) drop(q);
+                    }
+                    m &= keep;
+                    band &= keep;
+                    if (band) {
+                        // undecided: the reference distance on the float positions, a
+                        // global load.  A lane's first one counts as inside for now and
+                        // is decided after the scan, with one load round trip for the
+                        // whole wave; further ones are decided at once.
+                        if (pend < 0) {
+                            const int k = __builtin_ctz(band);
+                            band &= band - 1u;
+                            pend = nw * kWord + k;
+                            pq = q0 + k;
+                            m |= 1u << k;
+                        }
+                        while (band) {
+                            const int k = __builtin_ctz(band);
+                            band &= band - 1u;
+                            m |= (dist2_ref(pi, gpos[slot_of(q0 + k)], L, invL) < rcs2) ? (1u << k) : 0u;
+                        }
+                    }
+                    if (m) {
+                        if (nw < WP) {
+                            gm[nw * kTile] = m;
+                            gq[nw * kTile] = (unsigned short)q0;
+                            nw++;
+                        } else {
+                            over = 1;
+                        }
+                        cnt += __popc(m);
+                        const int s = q0 & 31;
+                        atomicOr(&s_used[q0 >> 5].x, m << s);
+                        const unsigned up = s ? m >> (32 - s) : 0u;
+                        if (up) atomicOr(&s_used[(q0 >> 5) + 1].x, up);
                     }
                 };
-                // the 27 cells in (dz, dy, dx) order; the three cells of a
-                // (dz, dy) row are consecutive union cells (hence one contiguous
-                // staged range) unless the window wraps that axis
+                // this part's rows of the 27 cells in (dz, dy, dx) order; the three
+                // cells of a (dz, dy) row are consecutive union cells (hence one
+                // contiguous staged range) unless the window wraps that axis
+                const int w0 = wmod(rx - 1 - sx, ex_), w1 = wmod(rx - sx, ex_), w2 = wmod(rx + 1 - sx, ex_);
+                const int r0 = part * (8 / SPLIT), r1 = part == SPLIT - 1 ? 9 : r0 + 8 / SPLIT;
                 #pragma unroll 1
-                for (int r = 0; r < 9; r++) {
-                    const int ua = s_wmap[win_of(3 * r)], ub = s_wmap[win_of(3 * r + 1)],
-                              uc = s_wmap[win_of(3 * r + 2)];
+                for (int r = r0; r < r1; r++) {
+                    const int iy = r % 3, iz = r / 3;
+                    // Only atoms within xr of this atom along x can be in the
+                    // list: the distance along y and z to the row's cells leaves
+                    // at most sqrt(rb2 - dy^2 - dz^2) along x, and the coarse x
+                    // difference is within one unit of the true one.  A row with
+                    // nothing left is skipped whole.
+                    const int dyb = (iy == 1) ? 0 : yb[iy >> 1], dzb = (iz == 1) ? 0 : zb[iz >> 1];
+                    const int rem = rb2 - dyb * dyb - dzb * dzb;
+                    if (rem < 0) continue;
+                    const int xr = (int)ceilf(sqrtf((float)rem)) + 2;
+                    const int wb = (wmod(rz + iz - 1 - sz, ez_) * ey_ + wmod(ry + iy - 1 - sy, ey_)) * ex_;
+                    const int ua = s_wmap[wb + w0], ub = s_wmap[wb + w1], uc = s_wmap[wb + w2];
                     if (ua >= nu || ub >= nu || uc >= nu) {  // every neighbor cell was marked; guard regardless
                         err |= ERR_INTERNAL;
                         continue;
                     }
                     const int4 A = s_cell[ua], B = s_cell[ub], Cc = s_cell[uc];
                     const bool one = ub == ua + 1 && uc == ub + 1;
-                    // Only atoms within xr of this atom along x can be in the
-                    // list: the distance along y and z to the row's cells leaves
-                    // at most sqrt(rb2 - dy^2 - dz^2) along x, and the coarse x
-                    // difference is within one unit of the true one.  A row with
-                    // nothing left is skipped whole.
-                    int xr = 0;
-                    if (trim) {
-                        const int dyb = (r % 3 == 1) ? 0 : yb[r % 3 >> 1], dzb = (r / 3 == 1) ? 0 : zb[r / 3 >> 1];
-                        const int rem = rb2 - dyb * dyb - dzb * dzb;
-                        if (rem < 0) continue;
-                        xr = (int)ceilf(sqrtf((float)rem)) + 2;
-                    }
-                    if (one) {
-                        int z = A.z, e = Cc.z + Cc.y;
-                        if (trim) {
-                            z = first_above(z, e, -xr - 1);
-                            e = first_above(z, e, xr);
-                        }
-                        scan_range(z, e);
-                    } else {
+                    // the outer cells' atoms within reach: from za in the first cell,
+                    // up to ec in the third
+                    const int za = first_above(A.z, A.z + A.y, -cell16, cell16 - xr - 1),
+                              ec = first_above(Cc.z, Cc.z + Cc.y, cell16, xr - cell16);
+                    #pragma unroll 1
+                    for (int k = 0; k < (one ? 1 : 3); k++) {
+                        const int z = k == 0 ? za : (k == 1 ? B.z : Cc.z);
+                        const int e = (one || k == 2) ? ec : (k == 0 ? A.z + A.y : B.z + B.y);
                         #pragma unroll 1
-                        for (int t = 0; t < 3; t++) {
-                            const int4 ce = t == 0 ? A : (t == 1 ? B : Cc);
-                            int z = ce.z, e = ce.z + ce.y;
-                            if (trim) {
-                                z = first_above(z, e, -xr - 1);
-                                e = first_above(z, e, xr);
+                        for (int q0 = z; q0 < e; q0 += kWord) word(q0, e - q0);
+                    }
+                }
+                if (pend >= 0 && !over) {  // the deferred candidate
+                    const bool in = dist2_ref(pi, gpos[slot_of(pq)], L, invL) < rcs2;
+                    if (!in) {
+                        const int w = pend / kWord;
+                        gm[w * kTile] &= ~(1u << (pend % kWord));
+                        cnt--;
+                    }
+                }
+            }
+            s_cnt[part][at] = cnt;
+            s_words[part][at] = (unsigned char)nw;
+            const int flag = (miss ? kMiss : 0) | (over ? kOver : 0);
+            if (flag) atomicOr(&s_flag, flag);
+            __syncthreads();
+            if (!d.idx16) {  // 32-bit rows share the area with the masks
+                int all = 0;
+#pragma unroll
+                for (int p = 0; p < SPLIT; p++) all += s_cnt[p][at];
+                if (all > kcap - kMaskRows - kLJTail) atomicOr(&s_flag, kOver);
+                __syncthreads();
+            }
+            if (s_flag & kOver) staged = false;
+        }
+        FMD_GLOBAL int* out = gmut(d.nbr) + (size_t)t.lt * d.kcap * kTile + lane;
+        // 16-bit rows of the global scan are built in the upper half of the
+        // tile's row area (which holds 2 kcap 16-bit entries per lane) and moved
+        // to the lower half by the placement below; 32-bit rows are built in place
+        FMD_GLOBAL unsigned short* out16 =
+            (FMD_GLOBAL unsigned short*)(gmut(d.nbr) + (size_t)t.lt * d.kcap * kTile) + (size_t)d.kcap * kTile + lane;
+        if (!staged) {
+            if (want_set) {  // the scan was given up: slots in the bonded tables too
+                if (valid) bonded(false);
+            }
+            cnt = 0;
+            nw = 0;
+            if (valid && part == 0) {
+                // global-memory scan with the same visiting order
+                auto key_of = [&](int c) {
+                    return (int)cell_key(wrap_cell(cx, c % 3 - 1, nx), wrap_cell(cy, (c / 3) % 3 - 1, nx),
+                                         wrap_cell(cz, c / 9 - 1, nx));
+                };
+                // bonded partners past the first four are read from the table
+                // (slots), which this lane wrote
+                const FMD_GLOBAL int* bt = gview(d.bnd) + (size_t)t.lt * d.bcap * kTile + lane;
+                for (int c = 0; c < 27; c++) {
+                    const int k = key_of(c);
+                    bool seen = false;
+                    if (nx < 3)
+                        for (int v = 0; v < c; v++) seen |= (key_of(v) == k);
+                    if (seen) continue;
+                    const int s0 = cstart[k], e0 = cstart[k + 1];
+                    for (int q0 = s0; q0 < e0; q0 += kBuildChunk) {
+                        float4 pj[kBuildChunk];
+#pragma unroll
+                        for (int k2 = 0; k2 < kBuildChunk; k2++) pj[k2] = gpos[min(q0 + k2, e0 - 1)];
+                        if (d.idx16)
+                            build_chunk<true>(pj, q0, e0 - q0, i, pi, L, invL, rcs2, ex, nb, d.bcap, bt, out, out16, kcap, cnt);
+                        else
+                            build_chunk<false>(pj, q0, e0 - q0, i, pi, L, invL, rcs2, ex, nb, d.bcap, bt, out, out16, kcap, cnt);
+                    }
+                }
+            }
+            __syncthreads();  // s_cnt is read by every part above
+            s_cnt[part][at] = cnt;
+            __syncthreads();
+        }
+        // Row lengths: start = this part's first entry, total over the parts
+        int start = 0, total = 0, wstart = 0, words = 0;
+#pragma unroll
+        for (int p = 0; p < SPLIT; p++) {
+            const int c = s_cnt[p][at], n = staged ? s_words[p][at] : 0;
+            start += p < part ? c : 0;
+            wstart += p < part ? n : 0;
+            total += c;
+            words += n;
+        }
+        if (words > kColWords || total > kcap) atomicOr(&s_flag, kMany);
+        const int stored = min(total, kcap);
+        const int padded = valid ? ((stored + kLJTail - 1) / kLJTail) * kLJTail : 0;
+        // Columns: the group's rows go to columns in descending order of their
+        // padded length (ties by slot; lengths from 252 up count as one), so the
+        // 64 rows a wave streams are of nearly equal length; gperm[column] names
+        // the atom.  A counting sort: rows of the same length in the wave by
+        // ballot, in the group through s_hist.
+        const int bucket = min(padded / kLJTail, 63);
+        int within = 0;
+        if (part == 0) {
+            unsigned long long todo = ~0ull;
+            while (todo) {
+                const int lead = __builtin_ctzll(todo);
+                const int b = __builtin_amdgcn_readlane(bucket, lead);
+                const unsigned long long same = __ballot(bucket == b);
+                if (bucket == b) within = lane_prefix(same);
+                if (lane == lead) s_hist[tl][b] = __popcll(same);
+                todo &= ~same;
+            }
+        }
+        if (staged && wv == kGroupTiles * SPLIT - 1) {
+            // used atoms before each word of the staged set
+            int base = 0;
+            for (int w0 = 0; w0 < kBuildStage / 32; w0 += 64) {
+                const int w = w0 + lane;
+                const int c = w < kBuildStage / 32 ? __popc(s_used[w].x) : 0;
+                int x = c;
+#pragma unroll
+                for (int o = 1; o < 64; o <<= 1) {
+                    const int y = __shfl_up(x, o, 64);
+                    if (lane >= o) x += y;
+                }
+                if (w < kBuildStage / 32) s_used[w].y = (unsigned)(base + x - c);
+                base += __shfl(x, 63, 64);
+            }
+            if (lane == 0) s_ncomp = base;
+        }
+        __syncthreads();
+        // the group's neighbor set: used staged atoms, every atom itself and its
+        // bonded partners (the force kernel reads them from the set too),
+        // numbered in staged (slot) order
+        const int ncomp = staged ? s_ncomp : 0;
+        const int flags = s_flag;
+        const bool compact = staged && want_set && ncomp <= kGroupStage && !(flags & kMiss);  // uniform
+        const bool bycol = compact && !(flags & kMany);
+        if (part == 0) {
+            int tot = 0;  // rows of length `lane` in the group, then of that length or more
+#pragma unroll
+            for (int w = 0; w < kGroupTiles; w++) tot += s_hist[w][lane];
+            int suf = tot;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int y = __shfl_down(suf, o, 64);
+                if (lane + o < 64) suf += y;
+            }
+            int rank = __shfl(suf - tot, bucket, 64) + within;
+#pragma unroll
+            for (int w = 0; w < kGroupTiles - 1; w++) rank += w < tl ? s_hist[w][bucket] : 0;
+            s_rank[at] = (unsigned short)rank;
+            gmut(d.gperm)[(size_t)grp * kGroupSlots + rank] = (unsigned char)at;
+            atomicMax(&s_tlen[rank / kTile], padded);
+        }
+        if (compact)
+            for (int q = tid; q < nstage; q += NT) {
+                const uint2 u = s_used[q >> 5];
+                if ((u.x >> (q & 31)) & 1u) {
+                    const int idx = (int)u.y + __popc(u.x & ((1u << (q & 31)) - 1u));
+                    const int slot = slot_of(q);
+                    const size_t p = (size_t)grp * kGroupStage + idx;
+                    s_cidx[q] = (unsigned short)(idx << 4);
+                    if (d.idx16) ((FMD_GLOBAL unsigned short*)gmut(d.gstage))[p] = (unsigned short)slot;
+                    else gmut(d.gstage)[p] = slot;
+                }
+            }
+        if (tid == 0) gmut(d.gcount)[grp] = compact ? ncomp : -1;
+        __syncthreads();
+        // every row of a wave is padded to the wave's longest, whose length the
+        // force pass reads as one uniform bound
+        const int rank = s_rank[at];
+        const int wpad = s_tlen[rank / kTile];
+        if (part == 0 && rank % kTile == 0) gmut(d.tlen)[grp * kGroupTiles + rank / kTile] = wpad;
+        int selfent = i;  // the padding entry: the atom itself (rejected by r^2 = 0)
+        if (valid && want_set) {
+            if (compact) {
+                // bonded entries of a staged group: LDS byte offsets of the partners
+                // in the set instead of staged indices (role and type bits kept)
+                if (do_bonds)
+                    for (int b = 0; b < min(nb, d.bcap); b++) {
+                        FMD_GLOBAL int* p = gmut(d.bnd) + ((size_t)t.lt * d.bcap + b) * kTile + lane;
+                        const int e = *p;
+                        *p = (int)s_cidx[e & kSlotMask] | (e & ~kSlotMask);
+                    }
+                if (do_angles)
+                    for (int a = 0, na = (gview(d.bhdr)[i] >> 8) & 0xFF; a < na; a++) {
+                        FMD_GLOBAL int2* p = gmut(d.ang) + ((size_t)t.lt * d.acap + a) * kTile + lane;
+                        const int ex1 = p->x, ex2 = p->y;
+                        p->x = (int)s_cidx[ex1 & kSlotMask] | (ex1 & ~kSlotMask);
+                        p->y = (int)s_cidx[ex2 & kSlotMask] | (ex2 & ~kSlotMask);
+                    }
+                selfent = (int)s_cidx[qself];
+            } else if (staged) {
+                bonded(false);
+            }
+        }
+        // Placement.  From the masks, each part from its first entry on: an
+        // entry is its atom's LDS byte offset in the set (or its slot when the set
+        // did not fit).
+        FMD_GLOBAL int* dtile = gmut(d.nbr) + (size_t)(grp * kGroupTiles + rank / kTile) * d.kcap * kTile;
+        if (bycol) {
+            // One lane per column, every lane at the same row entry: a pass stores a
+            // whole 128-byte row (with a lane per atom and a word at a time, the
+            // lanes' stores fall in as many rows as lanes).  The atoms' masks go to
+            // LDS by column; with SPLIT > 1 each part places a share of the rows.
+            for (int w = 0; w < nw; w++) {
+                s_m[(wstart + w) * kGroupSlots + rank] = gm[w * kTile];
+                s_q[(wstart + w) * kGroupSlots + rank] = gq[w * kTile];
+            }
+            if (part == 0) s_col[rank] = (unsigned)total | (unsigned)(valid ? selfent : 0) << 16;
+            __syncthreads();
+            const unsigned cc = s_col[at];
+            const int n = (int)(cc & 0xFFFFu), pad = (int)(cc >> 16);
+            const int wp = __builtin_amdgcn_readfirstlane(s_tlen[tl]);
+            const int share = ((wp / kLJTail + SPLIT - 1) / SPLIT) * kLJTail;
+            const int k0 = part * share, k1 = min(wp, k0 + share);
+            int left = n - k0;  // entries left in the row
+            const unsigned* pm = s_m + at;
+            const unsigned short* pq = s_q + at;
+            unsigned m = 0u;
+            int q0 = 0;
+            if (left > 0) {
+                int skip = k0;
+                m = *pm;
+                while (skip > 0) {  // to this part's first entry
+                    const int c = __popc(m);
+                    if (c > skip) {
+                        for (; skip > 0; skip--) m &= m - 1u;
+                    } else {
+                        skip -= c;
+                        pm += kGroupSlots;
+                        pq += kGroupSlots;
+                        m = *pm;
+                    }
+                }
+                q0 = *pq;
+            }
+            auto emit = [&](auto* dst) __attribute__((always_inline)) {
+                for (int k = k0; k < k1; k += kLJTail, dst += kLJTail * kTile) {
+                    int q[kLJTail];
+#pragma unroll
+                    for (int j = 0; j < kLJTail; j++) {
+                        q[j] = -1;
+                        if (left > j) {
+                            while (!m) {
+                                pm += kGroupSlots;
+                                pq += kGroupSlots;
+                                m = *pm;
+                                q0 = *pq;
                             }
-                            scan_range(z, e);
+                            q[j] = q0 + __builtin_ctz(m);
+                            m &= m - 1u;
                         }
                     }
-                }
-            };
-            if (d.idx16) scan_rows(BoolC<true>{});
-            else scan_rows(BoolC<false>{});
-            // the deferred candidate: one load for the wave; outside -> the atom's
-            // own entry (its staged index), which the force pass and the pair
-            // readout skip
-            if (pend >= 0) {
-                const int pos = pend >> 12, q = pend & 0xFFF;
-                const bool in = dist2_ref(pi, gpos[slot_of(q)], L, invL) < rcs2;
-                if (!in && pos < kcap) {
-                    if (d.idx16) out16[pos * kTile] = (unsigned short)qself;
-                    else out[pos * kTile] = qself;
-                }
-            }
-            if (qself < 0 || qself >= nstage) {
-                err |= ERR_INTERNAL;
-                qself = 0;
-            }
-        } else if (valid) {
-            // global-memory scan with the same visiting order
-            auto key_of = [&](int c) {
-                return (int)cell_key(wrap_cell(cx, c % 3 - 1, nx), wrap_cell(cy, (c / 3) % 3 - 1, nx),
-                                     wrap_cell(cz, c / 9 - 1, nx));
-            };
-            for (int c = 0; c < 27; c++) {
-                const int k = key_of(c);
-                bool seen = false;
-                if (nx < 3)
-                    for (int v = 0; v < c; v++) seen |= (key_of(v) == k);
-                if (seen) continue;
-                const int s0 = cstart[k], e0 = cstart[k + 1];
-                for (int q0 = s0; q0 < e0; q0 += kBuildChunk) {
-                    float4 pj[kBuildChunk];
+                    left -= kLJTail;
+                    int e[kLJTail];
 #pragma unroll
-                    for (int k2 = 0; k2 < kBuildChunk; k2++) pj[k2] = gpos[min(q0 + k2, e0 - 1)];
-                    if (d.idx16)
-                        build_chunk<true>(pj, q0, e0 - q0, i, pi, L, invL, rcs2, ex, nb, d.bcap, bt, out, out16,
-                                          kcap, cnt, q0, nullptr);
-                    else
-                        build_chunk<false>(pj, q0, e0 - q0, i, pi, L, invL, rcs2, ex, nb, d.bcap, bt, out, out16,
-                                           kcap, cnt, q0, nullptr);
+                    for (int j = 0; j < kLJTail; j++) e[j] = (int)s_cidx[max(q[j], 0)];
+#pragma unroll
+                    for (int j = 0; j < kLJTail; j++) dst[j * kTile] = q[j] >= 0 ? e[j] : pad;
                 }
-            }
-        }
-        const int stored = min(cnt, kcap);
-        const int padded = valid ? ((stored + kLJTail - 1) / kLJTail) * kLJTail : 0;
-        int selfent = i;  // the padding entry: the atom itself (rejected by r^2 = 0)
-        bool compact = false;
-        if (staged) {
-            // the group's neighbor set: used staged atoms, every atom itself and
-            // its bonded partners (the force kernel reads them from the set too),
-            // numbered in staged (slot) order
-            int pmiss = 0;
-            if (valid) {
-                s_used[qself] = 1;
-                const int hv = gview(d.bhdr)[i], nbk = hv & 0xFF, nak = (hv >> 8) & 0xFF;
-                const FMD_GLOBAL int2* at = gview(d.ang) + (size_t)t.lt * d.acap * kTile + lane;
-                for (int b = 0; b < nbk; b++) {
-                    const int q = partner_q(bt[b * kTile] & kSlotMask);
-                    if (q < 0) pmiss = 1;
-                    else s_used[q] = 1;
-                }
-                for (int a = 0; a < nak; a++) {
-                    const int2 e = at[a * kTile];
-                    const int q1 = partner_q(e.x & kSlotMask), q2 = partner_q(e.y & kSlotMask);
-                    if (q1 < 0 || q2 < 0) pmiss = 1;
-                    if (q1 >= 0) s_used[q1] = 1;
-                    if (q2 >= 0) s_used[q2] = 1;
-                }
-            }
-            // the scan's last reads of s_pj precede the s_cidx writes below
-            pmiss = __syncthreads_or(pmiss);
-            const int per = (nstage + kGroupSlots - 1) / kGroupSlots;
-            const int q0 = min(tid * per, nstage), q1 = min(q0 + per, nstage);
-            int c = 0;
-            for (int q = q0; q < q1; q++) c += s_used[q];
-            int ncomp = 0;
-            int idx = block_excl_scan(c, s_wsum, &ncomp);
-            compact = ncomp <= kGroupStage && !d.nostage && !pmiss;
-            for (int q = q0; q < q1; q++)
-                if (s_used[q]) {
-                    s_cidx[q] = (unsigned short)idx;
-                    if (compact) {
-                        const int4 ce = s_cell[s_seg[q]];
-                        const int slot = ce.x + q - ce.z;
-                        const size_t at = (size_t)grp * kGroupStage + idx;
-                        if (d.idx16) ((FMD_GLOBAL unsigned short*)gmut(d.gstage))[at] = (unsigned short)slot;
-                        else gmut(d.gstage)[at] = slot;
+            };
+            FMD_GLOBAL int* ctile = gmut(d.nbr) + (size_t)t.lt * d.kcap * kTile;
+            if (d.idx16) emit((FMD_GLOBAL unsigned short*)ctile + k0 * kTile + lane);
+            else emit(ctile + k0 * kTile + lane);
+        } else if (staged) {
+            if (total > kcap) {  // more hits than the row holds (an error): leave out the last ones
+                int room = max(0, kcap - start);
+                for (int w = 0; w < nw; w++) {
+                    unsigned m = gm[w * kTile], keep = 0u;
+                    for (; m && room > 0; room--) {
+                        keep |= m & (0u - m);
+                        m &= m - 1u;
                     }
-                    idx++;
+                    gm[w * kTile] = keep;
                 }
-            if (tid == 0) gmut(d.gcount)[grp] = compact ? ncomp : -1;
-        } else if (tid == 0) {
-            gmut(d.gcount)[grp] = -1;
-        }
-        // Placement: the group's rows go to columns in descending order of
-        // their padded length (ties by slot), so the 64 rows a wave streams
-        // are of nearly equal length; gperm[column] names the atom.  Rows are
-        // moved a band of kPlaceBand entries at a time (every read of a band
-        // precedes every write), mapping staged indices to LDS byte offsets
-        // (or to slots when the neighbor set did not fit).
-        s_len[tid] = padded;
-        __syncthreads();
-        if (valid && compact) {
-            selfent = (int)s_cidx[qself] << 4;
-            const int hv = gview(d.bhdr)[i], nbk = hv & 0xFF, nak = (hv >> 8) & 0xFF;
-            const FMD_GLOBAL int2* at = gview(d.ang) + (size_t)t.lt * d.acap * kTile + lane;
-            // bonded entries of a staged group: LDS byte offsets of the partners
-            // in the set instead of slots (role and type bits kept)
-            for (int b = 0; b < nbk; b++) {
-                const int e = bt[b * kTile];
-                gmut(d.bnd)[((size_t)t.lt * d.bcap + b) * kTile + lane] =
-                    ((int)s_cidx[partner_q(e & kSlotMask)] << 4) | (e & ~kSlotMask);
             }
-            for (int a = 0; a < nak; a++) {
-                const int2 e = at[a * kTile];
-                gmut(d.ang)[((size_t)t.lt * d.acap + a) * kTile + lane] =
-                    make_int2(((int)s_cidx[partner_q(e.x & kSlotMask)] << 4) | (e.x & ~kSlotMask),
-                              ((int)s_cidx[partner_q(e.y & kSlotMask)] << 4) | (e.y & ~kSlotMask));
+            auto emit = [&](auto* dst, auto set) __attribute__((always_inline)) {
+                auto entry = [&](int q) __attribute__((always_inline)) {
+                    return decltype(set)::value ? (int)s_cidx[q] : slot_of(min(q, nstage - 1));
+                };
+                dst += start * kTile;
+                unsigned m = nw > 0 ? gm[0] : 0u;
+                int q0 = nw > 0 ? gq[0] : 0;
+                for (int w = 0; w < nw; w++) {
+                    unsigned mn = 0u;
+                    int qn = 0;
+                    if (w + 1 < nw) { mn = gm[(w + 1) * kTile]; qn = gq[(w + 1) * kTile]; }
+                    // four hits per pass, their reads in flight together (the bit of a
+                    // missing one reads entry 31 and is not stored)
+                    auto* p = dst;
+                    dst += __popc(m) * kTile;
+                    while (m) {
+                        const unsigned m1 = m & (m - 1u), m2 = m1 & (m1 - 1u), m3 = m2 & (m2 - 1u);
+                        const int e0 = entry(q0 + __builtin_ctz(m)), e1 = entry(q0 + __builtin_ctz(m1 | 0x80000000u)),
+                                  e2 = entry(q0 + __builtin_ctz(m2 | 0x80000000u)),
+                                  e3 = entry(q0 + __builtin_ctz(m3 | 0x80000000u));
+                        p[0] = e0;
+                        if (m1) p[kTile] = e1;
+                        if (m2) p[2 * kTile] = e2;
+                        if (m3) p[3 * kTile] = e3;
+                        p += 4 * kTile;
+                        m = m3 & (m3 - 1u);
+                    }
+                    m = mn;
+                    q0 = qn;
+                }
+                if (part == SPLIT - 1) {
+                    const int end = min(total, kcap);
+                    for (int k = end; k < wpad; k++, dst += kTile) *dst = selfent;
+                }
+            };
+            if (d.idx16) {
+                FMD_GLOBAL unsigned short* dst = (FMD_GLOBAL unsigned short*)dtile + (rank % kTile);
+                if (compact) emit(dst, BoolC<true>{});
+                else emit(dst, BoolC<false>{});
+            } else {
+                FMD_GLOBAL int* dst = dtile + (rank % kTile);
+                if (compact) emit(dst, BoolC<true>{});
+                else emit(dst, BoolC<false>{});
             }
-        }
-        int rank = 0, maxpad = 0;
-        for (int b = 0; b < kGroupSlots; b++) {
-            const int lb = s_len[b];
-            rank += (lb > padded || (lb == padded && b < tid)) ? 1 : 0;
-            maxpad = max(maxpad, lb);
-        }
-        gmut(d.gperm)[(size_t)grp * kGroupSlots + rank] = (unsigned char)tid;
-        // every row of a wave is padded to the wave's longest (its first
-        // column's), whose length the force pass reads as one uniform bound
-        __syncthreads();  // every read of s_len above precedes the writes below
-        s_len[rank] = padded;
-        __syncthreads();
-        const int wpad = s_len[rank & ~(kTile - 1)];
-        if ((rank & (kTile - 1)) == 0) gmut(d.tlen)[grp * kGroupTiles + rank / kTile] = wpad;
-        auto entry = [&](int q) {  // a staged index or slot as the force kernel reads it
-            if (!staged) return q;
-            if (compact) return (int)s_cidx[q] << 4;
-            return s_cell[s_seg[q]].x + q - s_cell[s_seg[q]].z;
-        };
-        // 32-bit rows, in place: every read of a band precedes every write
-        auto place = [&](auto* src, auto* dst) {
+        } else if (d.idx16) {
+            // rows of the global scan, from this lane's row in the upper half to
+            // its column in the lower half: no entry is both read and written
+            FMD_GLOBAL unsigned short* dst = (FMD_GLOBAL unsigned short*)dtile + (rank % kTile);
+            if (part == 0)
+                for (int k = 0; k < wpad; k++)
+                    dst[k * kTile] = (unsigned short)(k < stored ? (int)out16[k * kTile] : selfent);
+        } else {
+            // in place: rows are moved a band of kPlaceBand entries at a time
+            // (every read of a band precedes every write)
+            FMD_GLOBAL int* dst = dtile + (rank % kTile);
+            int maxpad = 0;
+#pragma unroll
+            for (int w = 0; w < kGroupTiles; w++) maxpad = max(maxpad, s_tlen[w]);
             for (int k0 = 0; k0 < maxpad; k0 += kPlaceBand) {
                 int v[kPlaceBand];
 #pragma unroll
                 for (int e = 0; e < kPlaceBand; e++) {
                     const int k = k0 + e;
-                    v[e] = (k < stored) ? entry((int)src[k * kTile]) : selfent;
+                    v[e] = (part == 0 && k < stored) ? out[k * kTile] : selfent;
                 }
                 __syncthreads();
 #pragma unroll
                 for (int e = 0; e < kPlaceBand; e++)
-                    if (k0 + e < wpad) dst[(k0 + e) * kTile] = v[e];
+                    if (part == 0 && k0 + e < wpad) dst[(k0 + e) * kTile] = v[e];
                 __syncthreads();
             }
-        };
-        // destination column: the same addressing as out / out16 (tile base in int units)
-        FMD_GLOBAL int* dtile = gmut(d.nbr) + (size_t)(grp * kGroupTiles + rank / kTile) * d.kcap * kTile;
-        if (d.idx16) {
-            // from this lane's row in the upper half to its column in the lower
-            // half: no entry is both read and written, so no barriers
-            // (the next band's loads are in flight while a band is converted)
-            FMD_GLOBAL unsigned short* dst = (FMD_GLOBAL unsigned short*)dtile + (rank % kTile);
-            int cur[kPlaceBand], nxt[kPlaceBand];
-            auto load = [&](int k0, int (&to)[kPlaceBand]) {
-#pragma unroll
-                for (int e = 0; e < kPlaceBand; e++) to[e] = (k0 + e < stored) ? (int)out16[(k0 + e) * kTile] : 0;
-            };
-            load(0, cur);
-            for (int k0 = 0; k0 < wpad; k0 += kPlaceBand) {
-                if (k0 + kPlaceBand < wpad) load(k0 + kPlaceBand, nxt);
-#pragma unroll
-                for (int e = 0; e < kPlaceBand; e++) {
-                    const int k = k0 + e;
-                    if (k < wpad) dst[k * kTile] = (unsigned short)((k < stored) ? entry(cur[e]) : selfent);
-                }
-#pragma unroll
-                for (int e = 0; e < kPlaceBand; e++) cur[e] = nxt[e];
-            }
-        } else {
-            place(out, dtile + (rank % kTile));
         }
-        if (valid) {
-            if (cnt > kcap) err |= ERR_NBR_OVERFLOW;
+        if (valid && part == 0) {
+            if (total > kcap) err |= ERR_NBR_OVERFLOW;
             gmut(d.nnbr)[i] = stored;
         }
         err = wave_or(err);
@@ -2255,6 +2452,12 @@ static inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 // 4,000 tiles) in one pass, without thousands of waves that find no tile
 static constexpr int kStrideBlocks = 1024;
 static constexpr int kBuildBlocks = 8192;   // grid cap of the list-build workgroups (one group each)
+// Up to this many groups in the launch (one per CU) each group's scan is shared
+// by four waves a tile; with more the CUs are full anyway and four only add
+// barriers and a second group's wait.  Measured per step, four waves against
+// one: 2,000 beads 40.1 / 41.6 us, 30,000 44.4 / 45.4, 60,000 45.6 / 46.8,
+// 100,000 60.7 / 59.5, 250,000 80.6 / 75.3.
+static constexpr int kSplitGroups = 256;
 static constexpr int kForceListBlocks = 1280;  // workgroups of a listed force pass (five per CU; a multiple of kXcds)
 static_assert(kForceListBlocks % kXcds == 0, "the listed force pass splits its grid evenly over the XCDs");
 
@@ -2316,7 +2519,10 @@ void launch_build(const Launch& l, int max_blocks) {
     int gb = cdiv(l.ntl, kGroupTiles);
     const int cap = max_blocks > 0 ? max_blocks : kBuildBlocks;
     if (gb > cap) gb = cap;
-    k_build<<<gb, kGroupSlots, 0, l.stream>>>(l.descs, l.tiles, l.rlist, l.nrt);
+    if (cdiv(l.ntl, kGroupTiles) <= kSplitGroups)
+        k_build<4><<<gb, kGroupSlots * 4, 0, l.stream>>>(l.descs, l.tiles, l.rlist, l.nrt);
+    else
+        k_build<1><<<gb, kGroupSlots, 0, l.stream>>>(l.descs, l.tiles, l.rlist, l.nrt);
 }
 static void force_kernel(const Launch& l, int g, int block, int t0, int nt, int terms, int kick, int mode,
                          int sel) {
