@@ -36,6 +36,13 @@ constexpr int kForkBuildBlocks = 1024;
 
 int size_class(int natoms);
 
+// Largest replica for which the one-stream step's cell sort runs in the
+// workgroup that decides the rebuild.  Measured per step, five sort kernels
+// against it: 2,000 beads 39.9 / 31.5 us, 7,400 (NVT) 52.4 / 45.2, 16,000
+// 43.8 / 38.7, 20,000 42.9 / 41.4, 24,000 46.0 / 47.5, 40,000 45.1 / 52.9;
+// 48 replicas of 1,000 to 6,000 beads 79.2 / 70.2.
+constexpr int kSortInDecide = 20480;
+
 struct Replica {
     int id = -1;
     int natoms = 0, nslots = 0, ntiles = 0, cls = 0;
@@ -65,6 +72,8 @@ struct Batch {
     bool fork = false;        // the step builds lists beside the force pass (launch_step_seq)
     bool fork_known = false;
     int64_t steps_since_fork = 0;  // steps launched since that choice
+    bool wgsort = false;      // every replica's cell sort may run in one workgroup
+    int max_atoms = 0;        // of one replica
     std::vector<int> ord;     // host copy of d_reps
     void* block = nullptr;    // the arrays above, carved from one device block
     size_t block_bytes = 0;

@@ -724,6 +724,11 @@ Batch* Engine::batch_for(const std::vector<int>& ids_in) {
     for (int id : ord)
         for (int j = 0; j < reps_[id]->desc.nchunks; j++) chunks.push_back(Tile{id, j});
     b->nch = (int)chunks.size();
+    b->wgsort = true;
+    for (int id : ord) {
+        b->max_atoms = std::max(b->max_atoms, reps_[id]->natoms);
+        b->wgsort = b->wgsort && reps_[id]->desc.ncell_cap <= kWgSortKeys && reps_[id]->natoms <= kWgSortAtoms;
+    }
     if (ord.size() > (size_t)kMaxReplicas) {
         delete b;
         fail(FMD_ERR_ARG, "more than " + std::to_string(kMaxReplicas) + " systems in one batch");
@@ -822,8 +827,9 @@ void Engine::decide_fork(Batch& b, bool may_sync) {
 // beside the cost of the cross-stream waits and runs its steps in one stream.
 void Engine::launch_step_seq(Batch& b) {
     Launch l = launch_of(b);
+    const bool sort = !b.fork && b.wgsort && b.max_atoms <= kSortInDecide;
     launch_pre(l);
-    launch_decide(l);
+    launch_decide(l, sort);
     // the part [f0, f1) of each size class's tile range (whole groups) with
     // that class's tuned workgroup shape (adjacent classes of one shape in
     // one launch)
@@ -852,7 +858,8 @@ void Engine::launch_step_seq(Batch& b) {
         staying(FS_STAYING, kEarlyForce, 1.0);
         (void)hipStreamWaitEvent(stream_, ev_join_, 0);
     } else {
-        launch_rebuild(l, 0, 1);
+        if (sort) launch_build(l);
+        else launch_rebuild(l, 0, 1);
         staying(FS_ALL, 0.0, 1.0);
     }
     launch_boundary(l, BND_STEP);

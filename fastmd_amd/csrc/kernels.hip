@@ -344,15 +344,150 @@ __global__ void __launch_bounds__(256) k_pre(const RepDesc* __restrict__ descs,
 }
 
 // ---------------------------------------------------------------------------
-// per-replica rebuild decision (src/main.cu:486-496, skin_trigger.cuh:18-33)
+// The Morton-ordered cell sort (below, k_bin to k_gather) of one replica by one
+// workgroup of 1024 threads: the same order, in one kernel and with the cell
+// counts in LDS, two 16-bit counts a word (at most kWgSortKeys cell keys and
+// kWgSortAtoms atoms).  One CU moves the replica's state, so its time grows with
+// the atoms, while five kernels cost their launches on every step, rebuilding
+// or not (1.5 us each).
 // ---------------------------------------------------------------------------
+constexpr int kSortThreads = 1024;
+constexpr int kWgSortNear = 16384;
+// a 16-byte record of any of the state arrays, moved as it is
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+template <class T> __device__ inline FMD_GLOBAL f32x4* raw4(T* p) { return (FMD_GLOBAL f32x4*)p; }
+struct SortLds {
+    unsigned h[kWgSortKeys / 2];       // counts, then first slots, of keys 2k and 2k + 1
+    int wsum[kSortThreads / 64];
+    int sx[kWgSortNear];               // the atoms' x sort keys in cell order
+    unsigned lo[32];                   // lower bound floor(c 2^32 / nx) of each cell coordinate
+};
+__device__ void sort_wg(const RepDesc& d, int nx, float ics, int cbits, float Lp, SortLds& s) {
+    const int tid = threadIdx.x, n = d.natoms, nkeys = 1 << (3 * cbits), nw = max(nkeys >> 1, 1);
+    for (int j = tid; j < nw; j += kSortThreads) s.h[j] = 0u;
+    if (tid < nx) s.lo[tid] = (unsigned)(((unsigned long long)tid << 32) / (unsigned)nx);
+    __syncthreads();
+    const double sc = 4294967296.0 / (double)Lp;
+    // kB atoms per thread and pass, their loads in flight together
+    constexpr int kB = 4;
+    for (int i0 = tid; i0 < n; i0 += kB * kSortThreads) {
+        f32x4 r[kB], v[kB], im[kB];
+#pragma unroll
+        for (int k = 0; k < kB; k++) {
+            const int i = min(i0 + k * kSortThreads, n - 1);
+            r[k] = raw4(d.pos)[i];
+            v[k] = raw4(d.vel)[i];
+            im[k] = raw4(d.img)[i];
+        }
+#pragma unroll
+        for (int k = 0; k < kB; k++) {
+            const int i = i0 + k * kSortThreads;
+            if (i < n) {
+                const int cx = cell_coord(r[k].x, ics, nx);
+                const int key = (int)cell_key(cx, cell_coord(r[k].y, ics, nx), cell_coord(r[k].z, ics, nx));
+                const int sh = (key & 1) * 16;
+                gmut(d.rank)[i] = (int)((atomicAdd(&s.h[key >> 1], 1u << sh) >> sh) & 0xFFFFu);
+                gmut(d.cell_of)[i] = key;
+                gmut(d.sortx)[i] = (int)(fix_coord(r[k].x, sc) - s.lo[cx]);
+                raw4(d.tmp_pos)[i] = r[k];
+                raw4(d.tmp_vel)[i] = v[k];
+                raw4(d.tmp_img)[i] = im[k];
+            }
+        }
+    }
+    __syncthreads();
+    {  // exclusive scan of the counts; thread t holds the words [t per, (t + 1) per)
+        const int per = (nw + kSortThreads - 1) / kSortThreads, w0 = tid * per, lane = lane_id();
+        int sum = 0;
+        for (int w = w0; w < min(w0 + per, nw); w++) sum += (int)(s.h[w] & 0xFFFFu) + (int)(s.h[w] >> 16);
+        int x = sum;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(x, o, 64);
+            if (lane >= o) x += y;
+        }
+        if (lane == 63) s.wsum[tid >> 6] = x;
+        __syncthreads();
+        int run = x - sum;
+        for (int w = 0; w < (tid >> 6); w++) run += s.wsum[w];
+        for (int w = w0; w < min(w0 + per, nw); w++) {
+            const unsigned c = s.h[w];
+            const int a = run, b = run + (int)(c & 0xFFFFu);
+            run = b + (int)(c >> 16);
+            s.h[w] = (unsigned)a | (unsigned)b << 16;
+            gmut(d.cell_start)[2 * w] = a;
+            gmut(d.cell_start)[2 * w + 1] = b;
+        }
+        if (tid == 0) gmut(d.cell_start)[nkeys] = n;
+    }
+    __syncthreads();
+    auto first = [&](int key) { return (int)((s.h[key >> 1] >> ((key & 1) * 16)) & 0xFFFFu); };
+    const bool near = n <= kWgSortNear;  // the sort keys in LDS, else in order2
+    for (int i0 = tid; i0 < n; i0 += kB * kSortThreads) {
+        int key[kB], rk[kB], sx[kB];
+#pragma unroll
+        for (int k = 0; k < kB; k++) {
+            const int i = min(i0 + k * kSortThreads, n - 1);
+            key[k] = gview(d.cell_of)[i];
+            rk[k] = gview(d.rank)[i];
+            sx[k] = gview(d.sortx)[i];
+        }
+#pragma unroll
+        for (int k = 0; k < kB; k++) {
+            const int i = i0 + k * kSortThreads;
+            if (i < n) {
+                const int dst = first(key[k]) + rk[k];
+                gmut(d.order)[dst] = i;
+                if (near) s.sx[dst] = sx[k];
+                else gmut(d.order2)[dst] = sx[k];
+            }
+        }
+    }
+    __syncthreads();
+    // rank inside the cell by x, then global id, and the move to the final slot
+    auto sx = [&](int c) __attribute__((always_inline)) { return near ? s.sx[c] : gview(d.order2)[c]; };
+    auto move = [&](int q, int key, f32x4 p, f32x4 v, f32x4 im) __attribute__((always_inline)) {
+        const int b = first(key), e = key + 1 < nkeys ? first(key + 1) : n, rx = sx(q);
+        const int gid = __float_as_int(im[3]);
+        int to = b;
+        for (int c = b; c < e; c++) {
+            const int rc = sx(c);
+            to += (rc < rx) || (rc == rx && c != q && gview(d.tmp_img)[gview(d.order)[c]].w < gid);
+        }
+        raw4(d.pos)[to] = p;
+        raw4(d.pos_ref)[to] = p;
+        raw4(d.vel)[to] = v;
+        raw4(d.img)[to] = im;
+        gmut(d.gid)[to] = gid;
+        gmut(d.slot_of)[gid] = to;
+        raw4(d.ipos)[to] = f32x4{__uint_as_float(fix_coord(p.x, sc)), __uint_as_float(fix_coord(p.y, sc)),
+                                 __uint_as_float(fix_coord(p.z, sc)), p.w};
+    };
+    for (int q0 = tid; q0 < n; q0 += 2 * kSortThreads) {  // two atoms, their loads in flight together
+        const int q1 = q0 + kSortThreads;
+        const int s0 = gview(d.order)[q0], s1 = gview(d.order)[min(q1, n - 1)];
+        const int k0 = gview(d.cell_of)[s0], k1 = gview(d.cell_of)[s1];
+        const f32x4 p0 = raw4(d.tmp_pos)[s0], p1 = raw4(d.tmp_pos)[s1];
+        const f32x4 v0 = raw4(d.tmp_vel)[s0], v1 = raw4(d.tmp_vel)[s1];
+        const f32x4 m0 = raw4(d.tmp_img)[s0], m1 = raw4(d.tmp_img)[s1];
+        move(q0, k0, p0, v0, m0);
+        if (q1 < n) move(q1, k1, p1, v1, m1);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// per-replica rebuild decision (src/main.cu:486-496, skin_trigger.cuh:18-33),
+// with SORT also the cell sort of a replica that rebuilds
+// ---------------------------------------------------------------------------
+template <bool SORT>
 __global__ void __launch_bounds__(1024) k_decide(const RepDesc* __restrict__ descs,
                                                  const int* __restrict__ reps, int nr,
                                                  const int* __restrict__ rep_t0, int* __restrict__ rlist,
                                                  int* __restrict__ nrt) {
     __shared__ float s_max[16];
     __shared__ int s_bad[16];
-    __shared__ int s_base;
+    __shared__ int s_base, s_nx, s_cb;
+    __shared__ float s_ics, s_L;
     const RepDesc& d = descs[reps[blockIdx.x]];
     RepState* st = d.st;
     if (!st->active) return;
@@ -396,7 +531,12 @@ __global__ void __launch_bounds__(1024) k_decide(const RepDesc* __restrict__ des
                 st->maxdisp_bits = 0;
                 st->nrebuilds++;
                 set_grid(d, st);
-                s_base = atomicAdd(nrt, d.ntiles);  // this replica's run of the rebuild tile list
+                if (st->err) {  // the box outgrew the cell arrays: the replica has stopped
+                    st->rebuild = 0;
+                } else {
+                    s_nx = st->nx; s_cb = st->cbits; s_ics = st->inv_cs; s_L = st->Lp;
+                    s_base = atomicAdd(nrt, d.ntiles);  // this replica's run of the rebuild tile list
+                }
             } else {
                 st->since_rebuild = since;
                 st->maxdisp_bits = __float_as_int(md);
@@ -409,6 +549,10 @@ __global__ void __launch_bounds__(1024) k_decide(const RepDesc* __restrict__ des
     const int base = s_base;
     if (base >= 0)
         for (int k = threadIdx.x; k < d.ntiles; k += blockDim.x) rlist[base + k] = rep_t0[blockIdx.x] + k;
+    if constexpr (SORT) {
+        __shared__ SortLds s_sort;
+        if (base >= 0) sort_wg(d, s_nx, s_ics, s_cb, s_L, s_sort);
+    }
 }
 
 // Radius of gyration of each chain (src/analysis/rg.cu:3-69): unwrapped
@@ -2465,9 +2609,10 @@ void launch_pre(const Launch& l) {
     if (l.ntl <= 0) return;
     k_pre<<<cdiv(l.ntl, 4), 256, 0, l.stream>>>(l.descs, l.tiles, l.ntl, l.nrt);
 }
-void launch_decide(const Launch& l) {
+void launch_decide(const Launch& l, bool sort) {
     if (l.nr <= 0) return;
-    k_decide<<<l.nr, 1024, 0, l.stream>>>(l.descs, l.reps, l.nr, l.rep_t0, l.rlist, l.nrt);
+    if (sort) k_decide<true><<<l.nr, kSortThreads, 0, l.stream>>>(l.descs, l.reps, l.nr, l.rep_t0, l.rlist, l.nrt);
+    else k_decide<false><<<l.nr, kSortThreads, 0, l.stream>>>(l.descs, l.reps, l.nr, l.rep_t0, l.rlist, l.nrt);
 }
 void launch_rg(const RepDesc* d, int nchains, double* out, hipStream_t s) {
     if (nchains <= 0) return;

@@ -61,3 +61,33 @@ def test_many_groups_build_the_rows_of_few(fmd, engine, orc):
     assert np.array_equal(engine.pairs(alone), orc.pair_set(p4, L, np.float32(2.5) + np.float32(0.3)))
     for s in sids + [alone]:
         engine.remove(s)
+
+
+@pytest.mark.parametrize("n,L", [(3, 9.0), (257, 8.6), (1023, 10.6), (2049, 13.5), (16385, 27.0), (20480, 29.0), (20481, 29.0),
+                                 (900, 60.0), (900, 91.0)])
+def test_sort_in_one_workgroup(fmd, engine, orc, n, L):
+    """The cell sort in the deciding workgroup (up to 20,480 atoms and 32,768
+    cell keys) and by the five sort kernels (a batch with a replica above the
+    limits): the same bits, and the exact pair set."""
+    rng = np.random.default_rng(n)
+    m = int(np.ceil(n ** (1 / 3)))
+    g = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
+    x = (g * L / m + rng.uniform(0, 0.2, (n, 3))) % L
+    x[0] = 0.0
+    d = fmd.Desc(pos4_of(x), L, KG_LJ, vel=rng.standard_normal((n, 3)), seed=3, T=(1.0, 1.0))
+    big = int(np.ceil(90000 ** (1 / 3)))
+    gb = np.stack(np.meshgrid(*[np.arange(big)] * 3, indexing="ij"), -1).reshape(-1, 3) * 1.1
+    other = fmd.Desc(pos4_of(gb), big * 1.1, KG_LJ, vel=rng.standard_normal((len(gb), 3)))
+    a, b, c = engine.add(d), engine.add(d), engine.add(other)
+    engine.step(a, 43)
+    engine.step([b, c], 43)
+    for u, w in zip(engine.state(a), engine.state(b)):
+        assert np.array_equal(u, w)
+    assert np.array_equal(engine.pairs(a), engine.pairs(b))
+    assert engine.rebuilds(a) >= 3
+    engine.step(a, 20 - 3)  # to the step of a forced rebuild at the latest
+    engine.build_neighbors(a)
+    p4, _, _ = engine.state(a)
+    assert np.array_equal(engine.pairs(a), orc.pair_set(p4, np.float32(L), np.float32(2.5) + np.float32(0.3)))
+    for s in (a, b, c):
+        engine.remove(s)
