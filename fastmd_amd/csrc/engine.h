@@ -66,7 +66,8 @@ struct Batch {
     int* d_rlist = nullptr;   // compact rebuild tile list (ntl entries)
     int* d_nrt = nullptr;     // its length
     Tile* d_chunks = nullptr; // (replica, chunk of kChunkTiles tiles) list
-    int nch = 0;
+    int nch = 0, max_chunks = 0;
+    bool any_nh = false;      // a replica with a Nose-Hoover chain
     int4* d_status = nullptr; // per replica (err, active, step lo, step hi), d_reps order
     int* d_phase = nullptr;   // per replica, steps since its last list build (d_reps order)
     bool fork = false;        // the step builds lists beside the force pass (launch_step_seq)

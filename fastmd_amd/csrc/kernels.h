@@ -18,6 +18,8 @@ struct Launch {
     int* nrt;              // its length
     const Tile* chunks;    // (replica, chunk) list for the first reduction level
     int nch;
+    int max_chunks;        // of one replica
+    bool any_nh;           // a replica with a Nose-Hoover chain (partials on every step)
     hipStream_t stream;
 };
 

@@ -121,6 +121,7 @@ constexpr int kLJChunk = 8;      // neighbors per software-pipelined chunk (kcap
 constexpr int kLJTail = 4;       // rows are padded to multiples of this; a last chunk may be this short
 constexpr int kBuildChunk = 8;   // list-build candidates whose loads are issued together
 constexpr int kBndThreads = 256;  // workgroup of the per-replica boundary reduction
+constexpr int kFusedChunks = 4;   // chunks a replica may have to be summed by that workgroup alone
 
 #pragma clang fp contract(off)
 __device__ inline float sq3(float x, float y, float z) { return x * x + y * y + z * z; }
@@ -140,31 +141,43 @@ __device__ u32x4 struct_load_b128(__amdgpu_buffer_rsrc_t rsrc, unsigned vindex, 
 // FP64 Nose-Hoover chain (src/integrate/nose_hoover.cu:86-178 / :356-447) and
 // NPT barostat (src/integrate/nose_hoover.cu:185-305), one lane per replica.
 // ---------------------------------------------------------------------------
+// The chain's loops are unrolled to kMaxChain under uniform conditions, so its
+// variables are registers (indexed at run time they would live in scratch).
 __device__ double nh_chain(RepState* st, double KE, double kT, int natoms, double half_dt) {
     const int M = st->M;
     double xi[kMaxChain], v[kMaxChain], dd[kMaxChain];
+#pragma unroll
     for (int k = 0; k < kMaxChain; k++) { xi[k] = st->xi[k]; v[k] = st->vxi[k]; dd[k] = 0.0; }
     const double Nf = 3.0 * (double)natoms, Q1 = st->Q1, Qr = st->Qr;
     const double dt2 = half_dt, dt4 = 0.5 * half_dt, dt8 = 0.25 * half_dt;
     double T = 2.0 * KE / Nf;
     if (Q1 > 0.0) dd[0] = (Nf * T - Nf * kT) / Q1;
-    for (int ich = M - 1; ich > 0; ich--) {
-        double e = (ich + 1 < M) ? exp(-dt8 * v[ich + 1]) : 1.0;
-        v[ich] = (v[ich] * e + dd[ich] * dt4) * e;
-    }
+#pragma unroll
+    for (int ich = kMaxChain - 1; ich > 0; ich--)
+        if (ich < M) {
+            double e = 1.0;
+            if (ich + 1 < kMaxChain && ich + 1 < M) e = exp(-dt8 * v[min(ich + 1, kMaxChain - 1)]);
+            v[ich] = (v[ich] * e + dd[ich] * dt4) * e;
+        }
     double e0 = (M > 1) ? exp(-dt8 * v[1]) : 1.0;
     v[0] = (v[0] * e0 + dd[0] * dt4) * e0;
     double scale = exp(-dt2 * v[0]);
     T *= scale * scale;
     if (Q1 > 0.0) dd[0] = (Nf * T - Nf * kT) / Q1;
-    for (int k = 0; k < M; k++) xi[k] += dt2 * v[k];
+#pragma unroll
+    for (int k = 0; k < kMaxChain; k++)
+        if (k < M) xi[k] += dt2 * v[k];
     v[0] = (v[0] * e0 + dd[0] * dt4) * e0;
-    for (int ich = 1; ich < M; ich++) {
-        double e = (ich + 1 < M) ? exp(-dt8 * v[ich + 1]) : 1.0;
-        double Qp = (ich == 1) ? Q1 : Qr;
-        dd[ich] = (Qp * v[ich - 1] * v[ich - 1] - kT) / Qr;
-        v[ich] = (v[ich] * e + dd[ich] * dt4) * e;
-    }
+#pragma unroll
+    for (int ich = 1; ich < kMaxChain; ich++)
+        if (ich < M) {
+            double e = 1.0;
+            if (ich + 1 < kMaxChain && ich + 1 < M) e = exp(-dt8 * v[min(ich + 1, kMaxChain - 1)]);
+            double Qp = (ich == 1) ? Q1 : Qr;
+            dd[ich] = (Qp * v[ich - 1] * v[ich - 1] - kT) / Qr;
+            v[ich] = (v[ich] * e + dd[ich] * dt4) * e;
+        }
+#pragma unroll
     for (int k = 0; k < kMaxChain; k++) { st->xi[k] = xi[k]; st->vxi[k] = v[k]; }
     return scale;
 }
@@ -2311,20 +2324,16 @@ k_force(const RepDesc* __restrict__ descs, const Tile* __restrict__ tiles, int t
 // tiles of one replica in a fixed order (thread t takes tile t, then the DPP
 // wave sum, then the four waves in order), so a large replica's sum is spread
 // over many CUs.
-__global__ void __launch_bounds__(256) k_chunk(const RepDesc* __restrict__ descs,
-                                              const Tile* __restrict__ chunks, int nch, int mode) {
+// The sum of one chunk, by a workgroup of 256 threads, to out[0 .. kNumSum + 1].
+__device__ __forceinline__ void chunk_sum(const RepDesc& d, int chunk, double (*red)[4], double* out) {
     constexpr int kN = kNumSum + 2;
-    __shared__ double red[kN][4];
-    const Tile ch = chunks[blockIdx.x];
-    const RepDesc& d = descs[ch.rep];
-    if (mode == BND_STEP && (!d.st->active || (d.ensemble == 0 && !d.st->want_obs))) return;  // nothing to sum
-    const int tl = ch.lt * kChunkTiles + threadIdx.x;
+    const int tl = chunk * kChunkTiles + threadIdx.x;
     double a[kN];
 #pragma unroll
     for (int c = 0; c < kN; c++) a[c] = 0.0;
     if (tl < d.ntiles)
 #pragma unroll
-        for (int c = 0; c < kN; c++) a[c] = d.wpart[(size_t)tl * kNumPart + c];
+        for (int c = 0; c < kN; c++) a[c] = gview(d.wpart)[(size_t)tl * kNumPart + c];
 #pragma unroll
     for (int c = 0; c < kN; c++) a[c] = c < kNumSum ? wave_sum_last(a[c]) : wave_max_last(a[c]);
     if (lane_id() == 63)
@@ -2333,10 +2342,17 @@ __global__ void __launch_bounds__(256) k_chunk(const RepDesc* __restrict__ descs
     __syncthreads();
     if (threadIdx.x < kN) {
         const int c = threadIdx.x;
-        d.cpart[(size_t)ch.lt * kNumPart + c] =
-            c < kNumSum ? ((red[c][0] + red[c][1]) + red[c][2]) + red[c][3]
-                        : fmax(fmax(red[c][0], red[c][1]), fmax(red[c][2], red[c][3]));
+        out[c] = c < kNumSum ? ((red[c][0] + red[c][1]) + red[c][2]) + red[c][3]
+                             : fmax(fmax(red[c][0], red[c][1]), fmax(red[c][2], red[c][3]));
     }
+}
+__global__ void __launch_bounds__(256) k_chunk(const RepDesc* __restrict__ descs,
+                                              const Tile* __restrict__ chunks, int nch, int mode) {
+    __shared__ double red[kNumSum + 2][4];
+    const Tile ch = chunks[blockIdx.x];
+    const RepDesc& d = descs[ch.rep];
+    if (mode == BND_STEP && (!d.st->active || (d.ensemble == 0 && !d.st->want_obs))) return;  // nothing to sum
+    chunk_sum(d, ch.lt, red, d.cpart + (size_t)ch.lt * kNumPart);
 }
 
 // Multiple-tau correlator push (src/analysis/correlator.cu:33-92), by the
@@ -2414,12 +2430,15 @@ __global__ void __launch_bounds__(64) k_nh_chain_run(RepState* st, const double*
 __device__ int boundary_tail(const RepDesc& d, RepState* st, int mode, const double (*red)[kBndThreads / 64],
                              double* smp) {
     double tot[kNumSum + 2];
+#pragma unroll
     for (int c = 0; c < kNumSum + 2; c++) {
         tot[c] = 0.0;
+#pragma unroll
         for (int w = 0; w < kBndThreads / 64; w++) tot[c] = c < kNumSum ? tot[c] + red[c][w] : fmax(tot[c], red[c][w]);
     }
     const double pe = tot[0];
     double W[6], K[6];
+#pragma unroll
     for (int c = 0; c < 6; c++) { W[c] = tot[1 + c]; K[c] = tot[7 + c]; }
     const double KE = 0.5 * (K[0] + K[3] + K[5]);
     const bool reduced = !(mode == BND_STEP && d.ensemble == 0 && !st->want_obs);
@@ -2518,30 +2537,73 @@ __device__ int boundary_tail(const RepDesc& d, RepState* st, int mode, const dou
 // the scalar integrator work and records (boundary_tail), then the stress
 // correlator push on sample steps.
 // ---------------------------------------------------------------------------
+// The scalar part is one lane's chain of FP64 arithmetic: it works on a copy of
+// the replica's state in LDS, read and written back by the whole workgroup (one
+// trip to memory each way instead of one per dependent field).  With FUSED (a
+// batch of replicas of at most kFusedChunks chunks) the first reduction level
+// is done here too, chunk after chunk, instead of by a k_chunk launch: worth the
+// launch for one chunk, or for several where most steps sum nothing (no chain
+// reads the kinetic energy), but two chunks one after the other take longer
+// than the launch (30,000 beads NVT 50.4 us per step against 49.2).  Together
+// per step: 2,000 beads 31.5 -> 28.6 us, 30,000 44.5 -> 41.7, NPT 120,000
+// 72.1 -> 69.1, 48 small replicas 70.1 -> 63.2.
+template <bool FUSED>
 __global__ void __launch_bounds__(kBndThreads) k_boundary(const RepDesc* __restrict__ descs,
                                                           const int* __restrict__ reps, int nr, int mode) {
+    static_assert(kBndThreads == kChunkTiles, "a workgroup sums a chunk");
+    constexpr int kStWords = (int)(sizeof(RepState) / 4);
+    static_assert(sizeof(RepState) % 4 == 0 && kStWords <= kBndThreads, "one word of the state per thread");
     __shared__ double red[kNumSum + 2][kBndThreads / 64];
+    __shared__ double s_cp[FUSED ? kFusedChunks * kNumPart : 1];
     __shared__ double smp[6];
     __shared__ int push;
+    __shared__ __align__(16) char s_state[sizeof(RepState)];
     const RepDesc& d = descs[reps[blockIdx.x]];
-    RepState* st = d.st;
-    if (mode == BND_START) {
-        if (threadIdx.x == 0 && st->active && !st->pre_ready) start_step(d, st, st->step + 1);
+    RepState* const gst = d.st;
+    RepState* const st = (RepState*)s_state;
+    if (mode == BND_STEP && d.ensemble == 0 && !gst->want_obs) {  // uniform
+        // a Langevin step that records nothing reduced no partials (k_force): the
+        // step count and the next step's target only
+        if (threadIdx.x == 0 && gst->active) {
+            const int64_t cur = gst->step + 1, stop = gst->stop;
+            const int err = gst->err;
+            gst->v_pending = 1.0f;
+            gst->step = cur;
+            gst->rec_step = cur;
+            gst->kicked = cur < stop ? 1 : 0;
+            if (cur >= stop || err) {
+                gst->active = 0;
+                gst->pre_ready = 0;
+            } else {
+                start_step(d, gst, cur + 1);
+            }
+        }
         return;
     }
-    if (mode == BND_STEP && !st->active) return;
-    // fixed-order reduction: per-thread strided sums, wave shuffles, then the
-    // waves in order (the same order whatever else is in the batch)
-    // second level: lane l of a wave reads component l % 16 of chunk 4 w + l / 16
-    // (+ 4 x waves per pass), the chunks in a fixed order
-    {
-        // a Langevin step that records nothing reduced no partials (k_force)
-        const bool none = mode == BND_STEP && d.ensemble == 0 && !st->want_obs;
+    if (threadIdx.x < kStWords) ((int*)s_state)[threadIdx.x] = gview((const int*)gst)[threadIdx.x];
+    __syncthreads();
+    if (mode == BND_START ? !(st->active && !st->pre_ready) : mode == BND_STEP && !st->active) return;  // uniform
+    if (mode == BND_START) {
+        if (threadIdx.x == 0) {
+            start_step(d, st, st->step + 1);
+            push = 0;
+        }
+    } else {
+        // fixed-order reduction: per-thread strided sums, wave shuffles, then the
+        // waves in order (the same order whatever else is in the batch)
+        // second level: lane l of a wave reads component l % 16 of chunk 4 w + l / 16
+        // (+ 4 x waves per pass), the chunks in a fixed order
+        if constexpr (FUSED) {
+            for (int ck = 0; ck < d.nchunks; ck++) {
+                chunk_sum(d, ck, red, s_cp + ck * kNumPart);
+                __syncthreads();
+            }
+        }
         const int lane = lane_id(), wv = threadIdx.x >> 6, c = lane & 15;
         const bool mx = c >= kNumSum;  // the two maximum keys
         double a = 0.0;
-        for (int ck = 4 * wv + (lane >> 4); !none && ck < d.nchunks; ck += 4 * (kBndThreads / 64)) {
-            const double x = d.cpart[(size_t)ck * kNumPart + c];
+        for (int ck = 4 * wv + (lane >> 4); ck < d.nchunks; ck += 4 * (kBndThreads / 64)) {
+            const double x = FUSED ? s_cp[FUSED ? ck * kNumPart + c : 0] : d.cpart[(size_t)ck * kNumPart + c];
             a = mx ? fmax(a, x) : a + x;
         }
         double o = __shfl_xor(a, 16, 64);
@@ -2549,10 +2611,11 @@ __global__ void __launch_bounds__(kBndThreads) k_boundary(const RepDesc* __restr
         o = __shfl_xor(a, 32, 64);
         a = mx ? fmax(a, o) : a + o;
         if (lane < kNumSum + 2) red[lane][wv] = a;
+        __syncthreads();
+        if (threadIdx.x == 0) push = boundary_tail(d, st, mode, red, smp);
     }
     __syncthreads();
-    if (threadIdx.x == 0) push = boundary_tail(d, st, mode, red, smp);
-    __syncthreads();
+    if (threadIdx.x < kStWords) gmut((int*)gst)[threadIdx.x] = ((const int*)s_state)[threadIdx.x];
     if (push) corr_push(d.corr, smp);
 }
 
@@ -2697,8 +2760,12 @@ void launch_force_listed(const Launch& l, int kick, int mode) {
 }
 void launch_boundary(const Launch& l, int mode) {
     if (l.nr <= 0) return;
-    if (mode != BND_START && l.nch > 0) k_chunk<<<l.nch, 256, 0, l.stream>>>(l.descs, l.chunks, l.nch, mode);
-    k_boundary<<<l.nr, kBndThreads, 0, l.stream>>>(l.descs, l.reps, l.nr, mode);
+    if (mode == BND_START || l.max_chunks <= (l.any_nh ? 1 : kFusedChunks)) {
+        k_boundary<true><<<l.nr, kBndThreads, 0, l.stream>>>(l.descs, l.reps, l.nr, mode);
+        return;
+    }
+    if (l.nch > 0) k_chunk<<<l.nch, 256, 0, l.stream>>>(l.descs, l.chunks, l.nch, mode);
+    k_boundary<false><<<l.nr, kBndThreads, 0, l.stream>>>(l.descs, l.reps, l.nr, mode);
 }
 void launch_ref_cells(const RepDesc* d, int natoms, int* out, hipStream_t s) {
     if (natoms <= 0) return;
