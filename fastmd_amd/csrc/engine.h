@@ -68,6 +68,7 @@ struct Batch {
     Tile* d_chunks = nullptr; // (replica, chunk of kChunkTiles tiles) list
     int nch = 0, max_chunks = 0;
     bool any_nh = false;      // a replica with a Nose-Hoover chain
+    bool any_tab = false;     // a replica with tabulated pairs
     int4* d_status = nullptr; // per replica (err, active, step lo, step hi), d_reps order
     int* d_phase = nullptr;   // per replica, steps since its last list build (d_reps order)
     bool fork = false;        // the step builds lists beside the force pass (launch_step_seq)

@@ -368,6 +368,7 @@ constexpr int kSortThreads = 1024;
 constexpr int kWgSortNear = 16384;
 // a 16-byte record of any of the state arrays, moved as it is
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 template <class T> __device__ inline FMD_GLOBAL f32x4* raw4(T* p) { return (FMD_GLOBAL f32x4*)p; }
 struct SortLds {
     unsigned h[kWgSortKeys / 2];       // counts, then first slots, of keys 2k and 2k + 1
@@ -1872,9 +1873,8 @@ struct LJSum {
 };
 
 template <bool OBS, bool CAP, bool ONE_TYPE, bool W16, bool LDS>
-__device__ __forceinline__ LJSum lj_loop(const RepDesc& d, int lt, int lane, int i, int4 pi, float L,
+__device__ __forceinline__ LJSum lj_loop(const RepDesc& d, int lt, int lane, int nw, int4 pi, float L,
                                          const int4* sp) {
-    const int nw = __builtin_amdgcn_readfirstlane(d.tlen[lt]);  // uniform: the loop control is scalar
     // the tile's rows as a raw buffer: entry k of this lane sits at byte
     // (k * kTile + lane) * entry size; the row offset goes in the scalar
     // offset, so fetching the next chunk costs no vector address arithmetic
@@ -1977,11 +1977,11 @@ __device__ __forceinline__ LJSum lj_loop(const RepDesc& d, int lt, int lane, int
     return LJSum{gx * fu, gy * fu, gz * fu, pe, v0 * hu2, v1 * hu2, v2 * hu2, v3 * hu2, v4 * hu2, v5 * hu2};
 }
 
-#define LJ_ARGS d, t.lt, lane, i, pi, L, sp
+#define LJ_ARGS d, t.lt, lane, nw, pi, L, sp
 template <bool W16, bool LDS>
-__device__ __forceinline__ LJSum lj_variants(const RepDesc& d, const Tile& t, int lane, int i, int4 pi,
+__device__ __forceinline__ LJSum lj_variants(const RepDesc& d, const Tile& t, int lane, int nw, int4 pi,
                                              float L, bool obs, const int4* sp) {
-    const bool cap = d.fcap > 0.0f, one = d.ntypes == 1 && d.lj[0].x != 0.0f && d.lj[0].y != 0.0f;
+    const bool cap = d.fcap > 0.0f, one = d.lj_kf != 0.0f;  // set for one (eps, sigma), neither zero
     if (!cap && one)
         return obs ? lj_loop<true, false, true, W16, LDS>(LJ_ARGS) : lj_loop<false, false, true, W16, LDS>(LJ_ARGS);
     if (!cap)
@@ -1997,36 +1997,73 @@ __device__ __forceinline__ LJSum lj_variants(const RepDesc& d, const Tile& t, in
 // [rmin, rmax]: node k sits at rmin + k dr, k = (int)((r - rmin) / dr) clamped
 // to [0, n - 2], weight t = (r - (rmin + k dr)) / dr.  Half the pair energy and
 // half the pair virial go to this atom, as in the LJ loop.
-template <bool W16>
-__device__ __forceinline__ LJSum table_loop(const RepDesc& d, int lt, int lane, int i, int4 pi, float L, const int4* sp) {
+// What bounds it is the chain of loads of a pair (its entry, the neighbor, the
+// table of the types, the two nodes), so kTabChunk pairs go through each step
+// together, pairs that do not count included, the next ones' entries requested
+// meanwhile.
+constexpr int kTabChunk = 4;
+template <bool W16, bool LDS>
+__device__ __forceinline__ LJSum table_loop(const RepDesc& d, int lt, int lane, int i, int4 pi, float L,
+                                            const int4* sp) {
     const int nn = d.nnbr[i];
-    const int* nl = d.nbr + (size_t)lt * d.kcap * kTile + lane;
-    const unsigned short* nl16 = (const unsigned short*)(d.nbr + (size_t)lt * d.kcap * kTile) + lane;
+    const FMD_GLOBAL int* nl = gview(d.nbr) + (size_t)lt * d.kcap * kTile + lane;
+    const FMD_GLOBAL unsigned short* nl16 =
+        (const FMD_GLOBAL unsigned short*)(gview(d.nbr) + (size_t)lt * d.kcap * kTile) + lane;
     const float u = L * 2.3283064365386963e-10f;
     const GridCut gc = grid_cut(d.st);
-    const int* trow = d.tab_idx + pi.w * d.ntypes;
+    const FMD_GLOBAL int* trow = gview(d.tab_idx) + pi.w * d.ntypes;
+    // nodes k and k + 1 in one load (8-byte aligned)
+    typedef f32x4 f32x4_8 __attribute__((aligned(8)));
+    const FMD_GLOBAL char* fe = (const FMD_GLOBAL char*)gview(d.tab_fe);
     LJSum s{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int k = 0; k < nn; k++) {
-        const int j = W16 ? (int)nl16[k * kTile] : nl[k * kTile];
-        const int4 pj = sp ? sp[j >> 4] : d.ipos[j];  // LDS byte offset or slot
-        const int tb = trow[pj.w];
-        if (tb < 0) continue;
-        const float ax = grid_d(pi.x, pj.x), ay = grid_d(pi.y, pj.y), az = grid_d(pi.z, pj.z);
-        if (!grid_inside(grid_s(ax, ay, az, gc.lo_g), gc.span)) continue;
-        const float dx = ax * u, dy = ay * u, dz = az * u;
-        const float4 tp = d.tab_parm[tb];
-        const int2 tn = d.tab_no[tb];
-        const float r = fminf(fmaxf(sqrtf(sq3(dx, dy, dz)), tp.x), tp.y);
-        const int idx = min(max((int)((r - tp.x) * tp.w), 0), tn.x - 2);
-        const float t = (r - (tp.x + (float)idx * tp.z)) * tp.w;
-        const float2 p0 = d.tab_fe[tn.y + idx], p1 = d.tab_fe[tn.y + idx + 1];
-        const float fs = p0.x + t * (p1.x - p0.x);
-        const float e = p0.y + t * (p1.y - p0.y);
-        const float hx = 0.5f * fs * dx, hy = 0.5f * fs * dy, hz = 0.5f * fs * dz;
-        s.fx += fs * dx; s.fy += fs * dy; s.fz += fs * dz;
-        s.pe += 0.5f * e;
-        s.w0 += hx * dx; s.w1 += hx * dy; s.w2 += hx * dz;
-        s.w3 += hy * dy; s.w4 += hy * dz; s.w5 += hz * dz;
+    int nxt[kTabChunk];
+    auto fetch = [&](int k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < kTabChunk; k++) {
+            const int q = min(k0 + k, nn - 1);
+            nxt[k] = W16 ? (int)nl16[q * kTile] : nl[q * kTile];
+        }
+    };
+    if (nn > 0) fetch(0);
+    for (int k0 = 0; k0 < nn; k0 += kTabChunk) {
+        int tb[kTabChunk];
+        float r[kTabChunk], dx[kTabChunk], dy[kTabChunk], dz[kTabChunk];
+        unsigned in = 0u;
+#pragma unroll
+        for (int k = 0; k < kTabChunk; k++) {
+            // LDS byte offset or slot
+            const f32x4 v = LDS ? *(const f32x4*)((const char*)sp + nxt[k]) : raw4(d.ipos)[nxt[k]];
+            const float ax = grid_d(pi.x, __float_as_uint(v.x)), ay = grid_d(pi.y, __float_as_uint(v.y)),
+                        az = grid_d(pi.z, __float_as_uint(v.z));
+            in |= (k0 + k < nn && grid_inside(grid_s(ax, ay, az, gc.lo_g), gc.span)) ? 1u << k : 0u;
+            dx[k] = ax * u; dy[k] = ay * u; dz[k] = az * u;
+            tb[k] = trow[__float_as_int(v.w)];
+        }
+        if (k0 + kTabChunk < nn) fetch(k0 + kTabChunk);
+        f32x4 p[kTabChunk];
+        float t[kTabChunk];
+#pragma unroll
+        for (int k = 0; k < kTabChunk; k++) {
+            if (tb[k] < 0) in &= ~(1u << k);
+            const int tab = max(tb[k], 0);
+            const f32x4 tp = raw4(d.tab_parm)[tab];
+            const f32x2 tn = ((const FMD_GLOBAL f32x2*)gview(d.tab_no))[tab];  // (points, offset)
+            r[k] = fminf(fmaxf(sqrtf(sq3(dx[k], dy[k], dz[k])), tp.x), tp.y);
+            const int idx = min(max((int)((r[k] - tp.x) * tp.w), 0), __float_as_int(tn.x) - 2);
+            t[k] = (r[k] - (tp.x + (float)idx * tp.z)) * tp.w;
+            p[k] = *(const FMD_GLOBAL f32x4_8*)(fe + (size_t)(__float_as_int(tn.y) + idx) * 8);
+        }
+#pragma unroll
+        for (int k = 0; k < kTabChunk; k++)
+            if ((in >> k) & 1u) {
+                const float fs = p[k].x + t[k] * (p[k].z - p[k].x);
+                const float e = p[k].y + t[k] * (p[k].w - p[k].y);
+                const float hx = 0.5f * fs * dx[k], hy = 0.5f * fs * dy[k], hz = 0.5f * fs * dz[k];
+                s.fx += fs * dx[k]; s.fy += fs * dy[k]; s.fz += fs * dz[k];
+                s.pe += 0.5f * e;
+                s.w0 += hx * dx[k]; s.w1 += hx * dy[k]; s.w2 += hx * dz[k];
+                s.w3 += hy * dy[k]; s.w4 += hy * dz[k]; s.w5 += hz * dz[k];
+            }
     }
     return s;
 }
@@ -2060,8 +2097,15 @@ __device__ __forceinline__ float angle_atan2(float y, float x) {
 // (src/integrate/langevin.cu:109-130).  Writes force[i] = (F, pe_i) and 13
 // FP64 partials per wave: pe, virial[6], kinetic tensor[6] (after the kick).
 // ---------------------------------------------------------------------------
-template <int TERMS, bool LIST = false>
-__global__ void __launch_bounds__(kMaxBlockK) __attribute__((amdgpu_waves_per_eu(6, 8)))
+//
+// TAB includes the tabulated pairs, for batches with such a replica: they need
+// more registers than the 80 of six waves per SIMD, which the others keep.
+// 9,000 beads with a table on half the pairs: 97.4 us per step with the pairs
+// one after the other in the one kernel, 67.9 in this form (four at a time; two
+// 73, eight spill: 102); without the table code the others' kernel is also
+// shorter (128 uneven replicas 355 -> 350 us per step, NPT 120,000 68.3 -> 66.8).
+template <int TERMS, bool LIST = false, bool TAB = false>
+__global__ void __launch_bounds__(kMaxBlockK) __attribute__((amdgpu_waves_per_eu(TAB ? 4 : 6, 8)))
 k_force(const RepDesc* __restrict__ descs, const Tile* __restrict__ tiles, int t0, int ntl, int kick, int mode,
         int sel, const int* __restrict__ rlist, const int* __restrict__ nrt) {
     constexpr int terms = TERMS;
@@ -2073,14 +2117,18 @@ k_force(const RepDesc* __restrict__ descs, const Tile* __restrict__ tiles, int t
         const Tile t = tiles[w];
         const RepDesc& d = descs[t.rep];
         RepState* st = d.st;
-        if (mode == FM_STEP && !st->active) return;
-        if (sel == FS_STAYING && st->rebuild) return;
         const int lane = lane_id();
-        // this lane computes the atom whose row the list build placed in its column
         const int grp = t.lt / kGroupTiles;
-        const int i = grp * kGroupSlots + d.gperm[t.lt * kTile + lane];
+        // requested together, before the replica's flags are looked at
+        const int active = st->active, rebuild = st->rebuild;
+        const int perm = gview(d.gperm)[t.lt * kTile + lane];
+        const int nst = (terms & 1) ? gview(d.gcount)[grp] : -1;
+        const int nw = (terms & 1) ? __builtin_amdgcn_readfirstlane(gview(d.tlen)[t.lt]) : 0;  // uniform: scalar loop control
+        if (mode == FM_STEP && !active) return;
+        if (sel == FS_STAYING && rebuild) return;
+        // this lane computes the atom whose row the list build placed in its column
+        const int i = grp * kGroupSlots + perm;
         // stage the group's neighbor set (coalesced slot list, one 16-byte position each)
-        const int nst = (terms & 1) ? d.gcount[grp] : -1;
         if (nst >= 0) {
             const int nth = blockDim.x, last = nst - 1;
             const FMD_GLOBAL int4* gp = gview(d.ipos);
@@ -2118,17 +2166,19 @@ k_force(const RepDesc* __restrict__ descs, const Tile* __restrict__ tiles, int t
             if (terms & 1) {
                 LJSum a;
                 if (sp) {  // the array itself: its LDS address is a constant of the kernel
-                    if (d.idx16) a = lj_variants<true, true>(d, t, lane, i, pi, L, obs, s_pos);
-                    else a = lj_variants<false, true>(d, t, lane, i, pi, L, obs, s_pos);
+                    if (d.idx16) a = lj_variants<true, true>(d, t, lane, nw, pi, L, obs, s_pos);
+                    else a = lj_variants<false, true>(d, t, lane, nw, pi, L, obs, s_pos);
                 } else {
-                    if (d.idx16) a = lj_variants<true, false>(d, t, lane, i, pi, L, obs, sp);
-                    else a = lj_variants<false, false>(d, t, lane, i, pi, L, obs, sp);
+                    if (d.idx16) a = lj_variants<true, false>(d, t, lane, nw, pi, L, obs, sp);
+                    else a = lj_variants<false, false>(d, t, lane, nw, pi, L, obs, sp);
                 }
                 fx = a.fx; fy = a.fy; fz = a.fz; pe = a.pe;
                 w0 = a.w0; w1 = a.w1; w2 = a.w2; w3 = a.w3; w4 = a.w4; w5 = a.w5;
-                if (d.ntables) {
-                    const LJSum b = d.idx16 ? table_loop<true>(d, t.lt, lane, i, pi, L, sp)
-                                            : table_loop<false>(d, t.lt, lane, i, pi, L, sp);
+                if (TAB && d.ntables) {
+                    const LJSum b = sp ? (d.idx16 ? table_loop<true, true>(d, t.lt, lane, i, pi, L, s_pos)
+                                                  : table_loop<false, true>(d, t.lt, lane, i, pi, L, s_pos))
+                                       : (d.idx16 ? table_loop<true, false>(d, t.lt, lane, i, pi, L, sp)
+                                                  : table_loop<false, false>(d, t.lt, lane, i, pi, L, sp));
                     fx += b.fx; fy += b.fy; fz += b.fz; pe += b.pe;
                     w0 += b.w0; w1 += b.w1; w2 += b.w2; w3 += b.w3; w4 += b.w4; w5 += b.w5;
                 }
@@ -2736,7 +2786,7 @@ static void force_kernel(const Launch& l, int g, int block, int t0, int nt, int 
                          int sel) {
     const size_t lds = 0;
 #define FMD_FORCE_ARGS l.descs, l.tiles, t0, nt, kick, mode, sel, l.rlist, l.nrt
-    switch (terms & 7) {
+    switch ((terms & 7) | (l.any_tab && (terms & 1) ? 8 : 0)) {
         case 1: k_force<1><<<g, block, lds, l.stream>>>(FMD_FORCE_ARGS); break;
         case 2: k_force<2><<<g, block, lds, l.stream>>>(FMD_FORCE_ARGS); break;
         case 3: k_force<3><<<g, block, lds, l.stream>>>(FMD_FORCE_ARGS); break;
@@ -2744,6 +2794,10 @@ static void force_kernel(const Launch& l, int g, int block, int t0, int nt, int 
         case 5: k_force<5><<<g, block, lds, l.stream>>>(FMD_FORCE_ARGS); break;
         case 6: k_force<6><<<g, block, lds, l.stream>>>(FMD_FORCE_ARGS); break;
         case 7: k_force<7><<<g, block, lds, l.stream>>>(FMD_FORCE_ARGS); break;
+        case 9: k_force<1, false, true><<<g, block, lds, l.stream>>>(FMD_FORCE_ARGS); break;
+        case 11: k_force<3, false, true><<<g, block, lds, l.stream>>>(FMD_FORCE_ARGS); break;
+        case 13: k_force<5, false, true><<<g, block, lds, l.stream>>>(FMD_FORCE_ARGS); break;
+        case 15: k_force<7, false, true><<<g, block, lds, l.stream>>>(FMD_FORCE_ARGS); break;
         default: k_force<0><<<g, block, lds, l.stream>>>(FMD_FORCE_ARGS); break;
     }
 #undef FMD_FORCE_ARGS
@@ -2755,8 +2809,12 @@ void launch_force(const Launch& l, int t0, int nt, int block, int terms, int kic
 }
 void launch_force_listed(const Launch& l, int kick, int mode) {
     if (l.ntl <= 0) return;
-    k_force<7, true><<<kForceListBlocks, kGroupSlots, 0, l.stream>>>(l.descs, l.tiles, 0, 0, kick, mode, FS_ALL,
-                                                                      l.rlist, l.nrt);
+    if (l.any_tab)
+        k_force<7, true, true><<<kForceListBlocks, kGroupSlots, 0, l.stream>>>(l.descs, l.tiles, 0, 0, kick, mode,
+                                                                                FS_ALL, l.rlist, l.nrt);
+    else
+        k_force<7, true><<<kForceListBlocks, kGroupSlots, 0, l.stream>>>(l.descs, l.tiles, 0, 0, kick, mode, FS_ALL,
+                                                                          l.rlist, l.nrt);
 }
 void launch_boundary(const Launch& l, int mode) {
     if (l.nr <= 0) return;
