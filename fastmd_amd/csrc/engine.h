@@ -43,6 +43,10 @@ int size_class(int natoms);
 // 48 replicas of 1,000 to 6,000 beads 79.2 / 70.2.
 constexpr int kSortInDecide = 20480;
 
+// Readback goes through pinned host memory, this many atoms at a time.
+constexpr int kReadAtoms = 1 << 17;
+constexpr size_t kReadBytes = (size_t)kReadAtoms * 40;  // positions, velocities and image counts
+
 struct Replica {
     int id = -1;
     int natoms = 0, nslots = 0, ntiles = 0, cls = 0;
@@ -189,6 +193,15 @@ class Engine {
     Launch launch_of(const Batch& b) const;
     Launch launch_of(const Batch& b, hipStream_t s) const;
     int32_t read_state(Replica& r, RepState& s);
+    // Pinned host memory of at least n bytes (null: none to be had), kept by the
+    // engine and grown to at most 2 kReadBytes.
+    char* pinned(size_t n);
+    void reserve_read(int natoms);
+    // Launches `read` for each range of at most kReadAtoms global ids into one of
+    // two halves of the pinned buffer (of `per_atom` bytes an atom) and `take`s
+    // it from there while the next range is read.
+    template <class Read, class Take>
+    int32_t read_ranges(int natoms, size_t per_atom, hipStream_t s, Read&& read, Take&& take);
 
     int device_ = 0;
     bool init_ok_ = false;
@@ -196,6 +209,9 @@ class Engine {
     hipStream_t stream_ = nullptr;
     hipStream_t side_ = nullptr;  // system creation beside the main stream's launches
     hipStream_t aux_ = nullptr;   // a step's list rebuilds beside its force pass
+    char* pin_ = nullptr;         // readback buffer (pinned)
+    size_t pin_bytes_ = 0;
+    hipEvent_t ev_read_[2] = {nullptr, nullptr};
     hipEvent_t ev_fork_ = nullptr, ev_sorted_ = nullptr, ev_join_ = nullptr;
     double* scratch_ = nullptr;   // this device's scratch array (device address), or null
     bool defer_free_ = false;

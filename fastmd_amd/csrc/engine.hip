@@ -48,6 +48,8 @@ Engine::Engine(int device, uint64_t budget) : device_(device) {
     if (hip_check(hipEventCreateWithFlags(&ev_fork_, hipEventDisableTiming), "hipEventCreate")) return;
     if (hip_check(hipEventCreateWithFlags(&ev_join_, hipEventDisableTiming), "hipEventCreate")) return;
     if (hip_check(hipEventCreateWithFlags(&ev_sorted_, hipEventDisableTiming), "hipEventCreate")) return;
+    for (auto& ev : ev_read_)
+        if (hip_check(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "hipEventCreate")) return;
     size_t fr = 0, tot = 0;
     if (hip_check(hipMemGetInfo(&fr, &tot), "hipMemGetInfo")) return;
     budget_ = budget ? budget : (uint64_t)(0.9 * (double)fr);
@@ -84,6 +86,9 @@ Engine::~Engine() {
     if (stream_) (void)hipStreamDestroy(stream_);
     if (side_) (void)hipStreamDestroy(side_);
     if (aux_) (void)hipStreamDestroy(aux_);
+    if (pin_) (void)hipHostFree(pin_);
+    for (auto& ev : ev_read_)
+        if (ev) (void)hipEventDestroy(ev);
     if (ev_fork_) (void)hipEventDestroy(ev_fork_);
     if (ev_join_) (void)hipEventDestroy(ev_join_);
     if (ev_sorted_) (void)hipEventDestroy(ev_sorted_);
@@ -633,6 +638,7 @@ int32_t Engine::create_impl(const fmd_system_desc* d, int32_t* sys, int kmult, b
     }
     reps_[id] = R;
     in_use_ += r.bytes;
+    reserve_read(r.natoms);
     // prime: initial build + forces (src/main.cu:311-342)
     Batch* b = batch_for({id});
     if (!b) {
@@ -939,6 +945,53 @@ int32_t Engine::launch_steps(const std::vector<int>& ids, int64_t k, bool use_gr
 
 int32_t Engine::sync() { return hip_check(hipStreamSynchronize(stream_), "hipStreamSynchronize"); }
 
+char* Engine::pinned(size_t n) {
+    if (n <= pin_bytes_) return pin_;
+    size_t want = 256 << 10;
+    while (want < n) want *= 2;
+    want = std::min(want, std::max(n, 2 * kReadBytes));
+    if (pin_) (void)hipHostFree(pin_);
+    pin_ = nullptr;
+    pin_bytes_ = 0;
+    void* p = nullptr;
+    if (hip_check(hipHostMalloc(&p, want, hipHostMallocDefault), "hipHostMalloc")) return nullptr;
+    pin_ = (char*)p;
+    pin_bytes_ = want;
+    return pin_;
+}
+
+static size_t range_bytes(int natoms, size_t per_atom) {
+    return ((size_t)std::min(natoms, kReadAtoms) + 255) / 256 * 256 * per_atom;
+}
+// With the system, so that its first readback does not pay for the buffer; a
+// failure is reported by the readback that needs it.
+void Engine::reserve_read(int natoms) {
+    if (!pinned(range_bytes(natoms, 40) * (natoms > kReadAtoms ? 2 : 1) + 4096)) err_.clear();
+}
+
+template <class Read, class Take>
+int32_t Engine::read_ranges(int natoms, size_t per_atom, hipStream_t s, Read&& read, Take&& take) {
+    const int nr = (natoms + kReadAtoms - 1) / kReadAtoms;
+    const size_t half = range_bytes(natoms, per_atom);
+    char* buf = pinned(nr > 1 ? 2 * half : half);
+    if (!buf) return FMD_ERR_NOMEM;
+    int32_t rc = FMD_OK;
+    auto start = [&](int k) {
+        const int g0 = k * kReadAtoms;
+        read(g0, std::min(kReadAtoms, natoms - g0), buf + (k & 1) * half);
+        if (!rc) rc = hip_check(hipGetLastError(), "launch(read)");
+        if (!rc) rc = hip_check(hipEventRecord(ev_read_[k & 1], s), "record(read)");
+    };
+    start(0);
+    for (int k = 0; k < nr && !rc; k++) {
+        if (k + 1 < nr) start(k + 1);
+        if (!rc) rc = hip_check(hipEventSynchronize(ev_read_[k & 1]), "sync(read)");
+        if (!rc) take(k * kReadAtoms, std::min(kReadAtoms, natoms - k * kReadAtoms), buf + (k & 1) * half);
+    }
+    if (rc) (void)hipStreamSynchronize(s);  // no kernel writes to the buffer any more
+    return rc;
+}
+
 int32_t Engine::read_state(Replica& r, RepState& s) {
     return hip_check(hipMemcpy(&s, r.st, sizeof(RepState), hipMemcpyDeviceToHost), "read state");
 }
@@ -1167,20 +1220,30 @@ int32_t Engine::compute_forces(int32_t sys, uint32_t terms, float* f4, double* v
     Launch l = launch_of(*b);
     launch_force(l, 0, b->ntl, 256, (int)(terms & 7u), 0, FM_OBS);
     launch_boundary(l, BND_REDUCE);
-    int32_t rc = sync();
     RepState s;
-    if (!rc) rc = read_state(*r, s);
-    if (!rc && f4) {
-        const RepDesc& D = r->desc;
-        std::vector<float4> f(D.nslots);
-        std::vector<int4> img(D.nslots);
-        rc = hip_check(hipMemcpy(f.data(), D.force, f.size() * 16, hipMemcpyDeviceToHost), "copy force");
-        if (!rc) rc = hip_check(hipMemcpy(img.data(), D.img, img.size() * 16, hipMemcpyDeviceToHost), "copy img");
-        if (!rc)
-            for (int i = 0; i < D.natoms; i++) {
-                int g = img[i].w;
-                f4[4 * g] = f[i].x; f4[4 * g + 1] = f[i].y; f4[4 * g + 2] = f[i].z; f4[4 * g + 3] = f[i].w;
-            }
+    const RepDesc* dd = d_descs_ + sys;
+    const size_t head = (sizeof(RepState) + 255) / 256 * 256;
+    int32_t rc;
+    if (f4 && r->natoms <= kReadAtoms) {  // the state with the forces: one wait
+        char* b = pinned(head + (size_t)r->natoms * 16);
+        rc = b ? FMD_OK : FMD_ERR_NOMEM;
+        if (!rc) {
+            launch_read_force(dd, 0, r->natoms, (float*)(b + head), b, stream_);
+            rc = hip_check(hipGetLastError(), "launch(read)");
+        }
+        if (!rc) rc = sync();
+        if (!rc) {
+            std::memcpy(&s, b, sizeof(s));
+            std::memcpy(f4, b + head, (size_t)r->natoms * 16);
+        }
+    } else {
+        rc = sync();
+        if (!rc) rc = read_state(*r, s);
+        if (!rc && f4)
+            rc = read_ranges(
+                r->natoms, 16, stream_,
+                [&](int g0, int n, char* b) { launch_read_force(dd, g0, n, (float*)b, nullptr, stream_); },
+                [&](int g0, int n, char* b) { std::memcpy(f4 + 4 * (size_t)g0, b, (size_t)n * 16); });
     }
     if (!rc) {
         if (vir)
@@ -1203,24 +1266,24 @@ int32_t Engine::compute_forces(int32_t sys, uint32_t terms, float* f4, double* v
 int32_t Engine::get_state(int32_t sys, float* pos4, float* vel3, int32_t* img3, bool wait) {
     Replica* r = rep(sys);
     if (!r) return fail(FMD_ERR_ARG, "no such system");
-    const RepDesc& D = r->desc;
-    std::vector<float4> p(D.nslots), v(D.nslots);
-    std::vector<int4> img(D.nslots);
-    RepState s;
-    int32_t rc = wait ? sync() : FMD_OK;
-    if (!rc) rc = hip_check(hipMemcpy(p.data(), D.pos, p.size() * 16, hipMemcpyDeviceToHost), "copy pos");
-    if (!rc) rc = hip_check(hipMemcpy(v.data(), D.vel, v.size() * 16, hipMemcpyDeviceToHost), "copy vel");
-    if (!rc) rc = hip_check(hipMemcpy(img.data(), D.img, img.size() * 16, hipMemcpyDeviceToHost), "copy img");
-    if (!rc) rc = read_state(*r, s);
-    if (rc) return rc;
-    const float vs = s.v_pending;  // post-force scale not yet applied to vel[]
-    for (int i = 0; i < D.natoms; i++) {
-        int g = img[i].w;
-        if (pos4) { pos4[4 * g] = p[i].x; pos4[4 * g + 1] = p[i].y; pos4[4 * g + 2] = p[i].z; pos4[4 * g + 3] = p[i].w; }
-        if (vel3) { vel3[3 * g] = v[i].x * vs; vel3[3 * g + 1] = v[i].y * vs; vel3[3 * g + 2] = v[i].z * vs; }
-        if (img3) { img3[3 * g] = img[i].x; img3[3 * g + 1] = img[i].y; img3[3 * g + 2] = img[i].z; }
-    }
-    return FMD_OK;
+    // wait: behind the steps on the main stream; else (a finished replica, beside
+    // other replicas' steps) on the side stream
+    hipStream_t st = wait ? stream_ : side_;
+    if (!pos4 && !vel3 && !img3) return wait ? sync() : FMD_OK;
+    const RepDesc* dd = d_descs_ + sys;
+    // in a range of n atoms: positions, then velocities, then image counts
+    auto at = [](char* b, int n, int part) { return b + (size_t)((n + 255) / 256 * 256) * part; };
+    return read_ranges(
+        r->natoms, 40, st,
+        [&](int g0, int n, char* b) {
+            launch_read_atoms(dd, g0, n, pos4 ? (float*)b : nullptr, vel3 ? (float*)at(b, n, 16) : nullptr,
+                              img3 ? (int*)at(b, n, 28) : nullptr, st);
+        },
+        [&](int g0, int n, char* b) {
+            if (pos4) std::memcpy(pos4 + 4 * (size_t)g0, b, (size_t)n * 16);
+            if (vel3) std::memcpy(vel3 + 3 * (size_t)g0, at(b, n, 16), (size_t)n * 12);
+            if (img3) std::memcpy(img3 + 3 * (size_t)g0, at(b, n, 28), (size_t)n * 12);
+        });
 }
 
 int32_t Engine::get_box(int32_t sys, double* L, bool of_positions) {
@@ -1401,6 +1464,7 @@ int32_t Engine::resume(const void* buf, uint64_t size, int32_t* sys) {
     }
     reps_[id] = R;
     in_use_ += r.bytes;
+    reserve_read(r.natoms);
     *sys = id;
     return FMD_OK;
 }
@@ -1554,11 +1618,17 @@ int32_t Engine::drain_thermo(int32_t sys, fmd_thermo* out, int32_t cap, int32_t*
     }
     if (to - from > cap) to = from + cap;
     if (to <= from) return FMD_OK;
-    std::vector<ThermoRec> ring(r->thermo_cap);
-    rc = hip_check(hipMemcpy(ring.data(), r->desc.thermo, ring.size() * sizeof(ThermoRec), hipMemcpyDeviceToHost), "copy thermo");
+    // the unread records only: one run of the ring, or two
+    std::vector<ThermoRec> rows(to - from);
+    for (int64_t k = from; k < to && !rc;) {
+        const int64_t at = k % r->thermo_cap, run = std::min(to - k, r->thermo_cap - at);
+        rc = hip_check(hipMemcpy(rows.data() + (k - from), r->desc.thermo + at, run * sizeof(ThermoRec),
+                                 hipMemcpyDeviceToHost), "copy thermo");
+        k += run;
+    }
     if (rc) return rc;
     for (int64_t k = from; k < to; k++) {
-        const ThermoRec& t = ring[k % r->thermo_cap];
+        const ThermoRec& t = rows[k - from];
         fmd_thermo& o = out[*n];
         o.step = t.step; o.ke = t.ke; o.pe = t.pe; o.temp = t.temp;
         for (int c = 0; c < 6; c++) o.press[c] = t.press[c];

@@ -73,6 +73,11 @@ void launch_status(const Launch& l, int4* out);
 // Per replica of the list: steps since its last list build (-1: inactive).
 void launch_phase(const Launch& l, int* out);
 // Reference cell ids / Morton keys by global id for one replica.
+// Atoms [g0, g0 + n) by global id to pinned host memory (16-byte aligned; any
+// may be null): positions (4 floats each), velocities and image counts (3 each).
+void launch_read_atoms(const RepDesc* d, int g0, int n, float* pos, float* vel, int* img, hipStream_t s);
+// The same for forces (4 floats each), and the replica's RepState.
+void launch_read_force(const RepDesc* d, int g0, int n, float* force, void* state, hipStream_t s);
 void launch_ref_cells(const RepDesc* d, int natoms, int* out, hipStream_t s);
 void launch_morton_keys(const RepDesc* d, int natoms, uint32_t* out, hipStream_t s);
 
