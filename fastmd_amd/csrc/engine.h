@@ -70,7 +70,7 @@ struct Batch {
     int* d_rlist = nullptr;   // compact rebuild tile list (ntl entries)
     int* d_nrt = nullptr;     // its length
     Tile* d_chunks = nullptr; // (replica, chunk of kChunkTiles tiles) list
-    int nch = 0, max_chunks = 0;
+    int nch = 0, max_chunks = 0, max_keys = 0;
     bool any_nh = false;      // a replica with a Nose-Hoover chain
     bool any_tab = false;     // a replica with tabulated pairs
     int4* d_status = nullptr; // per replica (err, active, step lo, step hi), d_reps order

@@ -735,6 +735,7 @@ Batch* Engine::batch_for(const std::vector<int>& ids_in) {
         b->max_chunks = std::max(b->max_chunks, reps_[id]->desc.nchunks);
         b->any_nh = b->any_nh || reps_[id]->ensemble != FMD_LANGEVIN;
         b->any_tab = b->any_tab || reps_[id]->desc.ntables > 0;
+        b->max_keys = std::max(b->max_keys, reps_[id]->desc.ncell_cap);
         b->max_atoms = std::max(b->max_atoms, reps_[id]->natoms);
         b->wgsort = b->wgsort && reps_[id]->desc.ncell_cap <= kWgSortKeys && reps_[id]->natoms <= kWgSortAtoms;
     }
@@ -785,7 +786,7 @@ void Engine::free_batch(Batch* b) {
 
 Launch Engine::launch_of(const Batch& b) const { return launch_of(b, stream_); }
 Launch Engine::launch_of(const Batch& b, hipStream_t s) const {
-    return Launch{d_descs_, b.d_tiles, b.ntl, b.d_reps, b.nr, b.d_rep_t0, b.d_rlist, b.d_nrt, b.d_chunks, b.nch, b.max_chunks, b.any_tab, b.any_nh, s};
+    return Launch{d_descs_, b.d_tiles, b.ntl, b.d_reps, b.nr, b.d_rep_t0, b.d_rlist, b.d_nrt, b.d_chunks, b.nch, b.max_chunks, b.max_keys, b.any_tab, b.any_nh, s};
 }
 
 // Whether the batch's steps build lists beside the force pass: with enough

@@ -19,6 +19,7 @@ struct Launch {
     const Tile* chunks;    // (replica, chunk) list for the first reduction level
     int nch;
     int max_chunks;        // of one replica
+    int max_keys;          // cell keys, the largest capacity of one replica
     bool any_tab;          // a replica with tabulated pairs
     bool any_nh;           // a replica with a Nose-Hoover chain (partials on every step)
     hipStream_t stream;

@@ -756,59 +756,64 @@ __global__ void __launch_bounds__(256) k_bin(REBUILD_ARGS) {
     }
 }
 
-// Exclusive scan of the cell counts, one 1024-thread workgroup per replica;
-// the counts are cleared for the next rebuild.
+// Exclusive scan of the cell counts (k_scatter clears them for the next
+// rebuild).  Workgroup (replica, y) of 1024 threads scans kScanKeys keys, four
+// consecutive ones a thread, from the sum of all the counts before them, which
+// it forms itself, instead of one workgroup that carries the sum through all keys
+// (115 us for the 262,144 keys of 1M beads).  1M beads: 200.1 -> 195.5 us per step.
+constexpr int kScanKeys = 4096;
 __global__ void __launch_bounds__(1024) k_scan(const RepDesc* __restrict__ descs,
                                                const int* __restrict__ reps, int nr, int always) {
-    // chunks of 1024 x 4 keys: thread t holds keys 4t..4t+3 of the chunk
-    // (one 16-byte load; a wave covers 1 KB contiguous), block-wide scan,
-    // then the running offset carries to the next chunk
-    __shared__ int wsum[16];
-    __shared__ int carry;
+    __shared__ int wsum[16], wbase[16];
     const RepDesc& d = descs[reps[blockIdx.x]];
     RepState* st = d.st;
     if (!always && !(st->active && st->rebuild)) return;
     const int nkeys = 1 << (3 * st->cbits);
-    const int lane = lane_id(), wv = threadIdx.x >> 6;
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for (int base = 0; base < nkeys; base += 4 * 1024) {
-        const int c0 = base + 4 * threadIdx.x;
-        int4 v = make_int4(0, 0, 0, 0);
-        if (c0 + 3 < nkeys) {
-            v = *(const int4*)(d.cell_cnt + c0);
-        } else {
-            if (c0 < nkeys) v.x = d.cell_cnt[c0];
-            if (c0 + 1 < nkeys) v.y = d.cell_cnt[c0 + 1];
-            if (c0 + 2 < nkeys) v.z = d.cell_cnt[c0 + 2];
-        }
-        const int local = v.x + v.y + v.z + v.w;
-        int x = local;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int y = __shfl_up(x, o, 64);
-            if (lane >= o) x += y;
-        }
-        if (lane == 63) wsum[wv] = x;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            int acc = carry;
-            for (int k = 0; k < 16; k++) { const int t = wsum[k]; wsum[k] = acc; acc += t; }
-            carry = acc;
-        }
-        __syncthreads();
-        const int run = wsum[wv] + x - local;  // exclusive prefix of this thread's keys
-        if (c0 + 3 < nkeys) {
-            *(int4*)(d.cell_start + c0) = make_int4(run, run + v.x, run + v.x + v.y, run + v.x + v.y + v.z);
-            *(int4*)(d.cell_cnt + c0) = make_int4(0, 0, 0, 0);
-        } else {
-            if (c0 < nkeys) { d.cell_start[c0] = run; d.cell_cnt[c0] = 0; }
-            if (c0 + 1 < nkeys) { d.cell_start[c0 + 1] = run + v.x; d.cell_cnt[c0 + 1] = 0; }
-            if (c0 + 2 < nkeys) { d.cell_start[c0 + 2] = run + v.x + v.y; d.cell_cnt[c0 + 2] = 0; }
-        }
-        __syncthreads();  // wsum is rewritten by the next chunk
+    const int k0 = blockIdx.y * kScanKeys;
+    if (k0 >= nkeys) return;
+    const int lane = lane_id(), wv = threadIdx.x >> 6, c0 = k0 + 4 * threadIdx.x;
+    const FMD_GLOBAL int* cnt = gview(d.cell_cnt);
+    typedef int i32x4 __attribute__((ext_vector_type(4)));
+    int before = 0;  // k0 is a multiple of kScanKeys: whole 16-byte loads
+#pragma unroll 4
+    for (int k = 4 * threadIdx.x; k < k0; k += kScanKeys) {
+        const i32x4 v = *(const FMD_GLOBAL i32x4*)(cnt + k);
+        before += v.x + v.y + v.z + v.w;
     }
-    if (threadIdx.x == 0) d.cell_start[nkeys] = carry;
+    int v[4] = {0, 0, 0, 0};
+    if (c0 + 3 < nkeys) {
+        const i32x4 q = *(const FMD_GLOBAL i32x4*)(cnt + c0);
+        v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+    } else {
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if (c0 + k < nkeys) v[k] = cnt[c0 + k];
+    }
+    const int local = v[0] + v[1] + v[2] + v[3];
+    int x = local;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
+        before += __shfl_xor(before, o, 64);
+    }
+    if (lane == 63) wsum[wv] = x;
+    if (lane == 0) wbase[wv] = before;
+    __syncthreads();
+    int run = x - local;
+#pragma unroll
+    for (int w = 0; w < 16; w++) run += wbase[w] + (w < wv ? wsum[w] : 0);
+    FMD_GLOBAL int* out = gmut(d.cell_start) + c0;
+    if (c0 + 3 < nkeys) {
+        *(FMD_GLOBAL i32x4*)out = i32x4{run, run + v[0], run + v[0] + v[1], run + v[0] + v[1] + v[2]};
+    } else {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if (c0 + k < nkeys) out[k] = run;
+            run += v[k];
+        }
+    }
+    if (c0 < nkeys && c0 + 4 >= nkeys) gmut(d.cell_start)[nkeys] = d.natoms;
 }
 
 __global__ void __launch_bounds__(256) k_scatter(REBUILD_ARGS) {
@@ -821,6 +826,9 @@ __global__ void __launch_bounds__(256) k_scatter(REBUILD_ARGS) {
             d.tmp_vel[i] = d.vel[i];
             d.tmp_img[i] = d.img[i];
         }
+        // the tile's share of the cell counts, cleared for the next rebuild
+        const int nkeys = 1 << (3 * st->cbits), per = (nkeys + d.ntiles - 1) / d.ntiles;
+        for (int k = t.lt * per + lane_id(); k < min((t.lt + 1) * per, nkeys); k += kTile) d.cell_cnt[k] = 0;
     }
 }
 
@@ -2809,7 +2817,7 @@ void launch_rebuild(const Launch& l, int always, int build) {
     int g = cdiv(l.ntl, 4);
     if (g > kStrideBlocks) g = kStrideBlocks;
     k_bin<<<g, 256, 0, l.stream>>>(l.descs, l.tiles, l.rlist, l.nrt);
-    k_scan<<<l.nr, 1024, 0, l.stream>>>(l.descs, l.reps, l.nr, always);
+    k_scan<<<dim3(l.nr, cdiv(l.max_keys, kScanKeys)), 1024, 0, l.stream>>>(l.descs, l.reps, l.nr, always);
     k_scatter<<<g, 256, 0, l.stream>>>(l.descs, l.tiles, l.rlist, l.nrt);
     k_rank<<<g, 256, 0, l.stream>>>(l.descs, l.tiles, l.rlist, l.nrt);
     k_gather<<<g, 256, 0, l.stream>>>(l.descs, l.tiles, l.rlist, l.nrt);
