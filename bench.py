@@ -457,7 +457,7 @@ def main():
         "roofline": {"bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": ach / HBM_PEAK_GBS, "traffic": traffic,
                      "traffic_source": os.path.relpath(TRAFFIC_PROFILE, ROOT) if traffic else None,
-                     "kernel": "k_force<1, false> (LJ over the Verlet list)", "ms_per_launch": ms_lj,
+                     "kernel": "k_force<1, false, false> (LJ over the Verlet list)", "ms_per_launch": ms_lj,
                      "alg_bytes_per_launch": bytes_lj, "stored_bytes_per_launch": stored_lj,
                      "listed_pairs": pairs,
                      "alg_bytes_rule": "36 B per bead + 4 B per listed pair (rows stored as 16-bit slots)",

@@ -25,7 +25,8 @@ constexpr int64_t kForkRecheck = 50 * kRebuildEvery;  // steps between two choic
 // share of the staying replicas' force pass launched beside the cell sort,
 // before the list build is queued (measured on 255 staggered replicas: 0.15,
 // 0.3, 0.5, 0.6, 0.7 and 0.85 gave 0.737, 0.730, 0.716, 0.723, 0.738 and
-// 0.774 ms per step, 0.740 without this part)
+// 0.774 ms per step, 0.740 without this part; with the list build placing hit
+// masks, 256 replicas, 0.35, 0.5, 0.65 and 0.8: 0.640, 0.632, 0.633 and 0.642)
 constexpr double kEarlyForce = 0.5;
 // workgroups of the list build in that step, the GPU's slots for it (256 CUs x
 // 4): the rebuilding replicas hold about a twentieth of the groups, and

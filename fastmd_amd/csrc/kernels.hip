@@ -8,8 +8,10 @@
 //
 // Step sequence (src/main.cu:403-630, one launch each, all replicas at once):
 //   pre       kick + drift (+ Langevin O step, NH/NPT scaling), wrap, skin max
-//   decide    per replica: rebuild if max displacement > (skin/2)^2 or every 20
-//   bin/scan/scatter/rank/gather   Morton-ordered cell sort (rebuilding only)
+//   decide    per replica: rebuild if max displacement > (skin/2)^2 or every 20;
+//             small replicas also sort their atoms here
+//   bin/scan/scatter/rank/gather   Morton-ordered cell sort of the larger ones
+//             (rebuilding only)
 //   build     Verlet list + bonded slot tables (rebuilding only)
 //   force     LJ + FENE/WCA + angle, post-force kick, FP64 wave partials
 //   boundary  per replica: FP64 reductions, NH chain / barostat, thermo record
