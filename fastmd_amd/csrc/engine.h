@@ -41,7 +41,8 @@ int size_class(int natoms);
 // workgroup that decides the rebuild.  Measured per step, five sort kernels
 // against it: 2,000 beads 39.9 / 31.5 us, 7,400 (NVT) 52.4 / 45.2, 16,000
 // 43.8 / 38.7, 20,000 42.9 / 41.4, 24,000 46.0 / 47.5, 40,000 45.1 / 52.9;
-// 48 replicas of 1,000 to 6,000 beads 79.2 / 70.2.
+// 48 replicas of 1,000 to 6,000 beads 79.2 / 70.2.  (Four kernels, 1.5 us less,
+// since k_rank moves the atoms; the crossing stays between 16,000 and 24,000.)
 constexpr int kSortInDecide = 20480;
 
 // Readback goes through pinned host memory, this many atoms at a time.

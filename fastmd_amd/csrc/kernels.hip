@@ -10,7 +10,7 @@
 //   pre       kick + drift (+ Langevin O step, NH/NPT scaling), wrap, skin max
 //   decide    per replica: rebuild if max displacement > (skin/2)^2 or every 20;
 //             small replicas also sort their atoms here
-//   bin/scan/scatter/rank/gather   Morton-ordered cell sort of the larger ones
+//   bin/scan/scatter/rank   Morton-ordered cell sort of the larger ones
 //             (rebuilding only)
 //   build     Verlet list + bonded slot tables (rebuilding only)
 //   force     LJ + FENE/WCA + angle, post-force kick, FP64 wave partials
@@ -359,7 +359,7 @@ __global__ void __launch_bounds__(256) k_pre(const RepDesc* __restrict__ descs,
 }
 
 // ---------------------------------------------------------------------------
-// The Morton-ordered cell sort (below, k_bin to k_gather) of one replica by one
+// The Morton-ordered cell sort (below, k_bin to k_rank) of one replica by one
 // workgroup of 1024 threads: the same order, in one kernel and with the cell
 // counts in LDS, two 16-bit counts a word (at most kWgSortKeys cell keys and
 // kWgSortAtoms atoms).  One CU moves the replica's state, so its time grows with
@@ -842,6 +842,13 @@ __global__ void __launch_bounds__(256) k_scatter(REBUILD_ARGS) {
 // compares grid coordinates modulo 2^32, and a position a rounding step
 // outside [0, L) (at -0 or L itself) stands at the cell's end where the grid
 // coordinate puts it.
+//
+// The atom is moved to its slot here, from k_scatter's copy.  The stores land
+// permuted within each cell, so they fill their lines less evenly than those of
+// a kernel of its own that goes by the new slots, but that kernel is a launch
+// in every step and reads the copy and the order once more.  Per step against
+// it: 30,000 beads 40.4 -> 38.9 us, 60,000 41.4 -> 39.7, 250,000 72.2 -> 70.4,
+// 1M 195.3 -> 193.8, 128 uneven replicas that rebuild together 355 -> 345.
 __global__ void __launch_bounds__(256) k_rank(REBUILD_ARGS) {
     REBUILD_LOOP {
         REBUILD_PROLOGUE
@@ -857,27 +864,18 @@ __global__ void __launch_bounds__(256) k_rank(REBUILD_ARGS) {
                 const int ro = d.sortx[o];
                 r += (ro < rx) || (ro == rx && d.tmp_img[o].w < g);
             }
-            d.order2[s + r] = src;
-        }
-    }
-}
-
-__global__ void __launch_bounds__(256) k_gather(REBUILD_ARGS) {
-    REBUILD_LOOP {
-        REBUILD_PROLOGUE
-        if (i < d.natoms) {
-            const int src = d.order2[i];
+            const int dst = s + r;
             const float4 p = d.tmp_pos[src];
             const int4 im = d.tmp_img[src];
-            d.pos[i] = p;
-            d.pos_ref[i] = p;
-            d.vel[i] = d.tmp_vel[src];
-            d.img[i] = im;
-            d.gid[i] = im.w;
-            d.slot_of[im.w] = i;
+            d.pos[dst] = p;
+            d.pos_ref[dst] = p;
+            d.vel[dst] = d.tmp_vel[src];
+            d.img[dst] = im;
+            d.gid[dst] = im.w;
+            d.slot_of[im.w] = dst;
             const double sc = 4294967296.0 / (double)st->Lp;
-            d.ipos[i] = make_int4((int)fix_coord(p.x, sc), (int)fix_coord(p.y, sc), (int)fix_coord(p.z, sc),
-                                  __float_as_int(p.w));
+            d.ipos[dst] = make_int4((int)fix_coord(p.x, sc), (int)fix_coord(p.y, sc), (int)fix_coord(p.z, sc),
+                                    __float_as_int(p.w));
         }
     }
 }
@@ -2822,7 +2820,6 @@ void launch_rebuild(const Launch& l, int always, int build) {
     k_scan<<<dim3(l.nr, cdiv(l.max_keys, kScanKeys)), 1024, 0, l.stream>>>(l.descs, l.reps, l.nr, always);
     k_scatter<<<g, 256, 0, l.stream>>>(l.descs, l.tiles, l.rlist, l.nrt);
     k_rank<<<g, 256, 0, l.stream>>>(l.descs, l.tiles, l.rlist, l.nrt);
-    k_gather<<<g, 256, 0, l.stream>>>(l.descs, l.tiles, l.rlist, l.nrt);
     if (build) launch_build(l);
 }
 void launch_build(const Launch& l, int max_blocks) {
