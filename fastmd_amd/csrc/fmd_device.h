@@ -173,8 +173,8 @@ struct RepDesc {
     int* cell_of;
     int* rank;
     int* sortx;            // [nslots] x grid coordinate relative to the atom's cell (the within-cell sort key)
-    int* order;
-    int* order2;
+    int* order;            // [nslots] sort scratch, in cell order: the atoms' cell keys (or their slots)
+    int* order2;           // [nslots] and their sort keys
     int* slot_of;          // [natoms] global id -> slot
     int* cell_cnt;         // [ncell_cap]
     int* cell_start;       // [ncell_cap + 1]

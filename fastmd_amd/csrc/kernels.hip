@@ -818,15 +818,21 @@ __global__ void __launch_bounds__(1024) k_scan(const RepDesc* __restrict__ descs
     if (c0 < nkeys && c0 + 4 >= nkeys) gmut(d.cell_start)[nkeys] = d.natoms;
 }
 
+// Atoms, their keys (order) and sort keys (order2) stored in cell order, a
+// cell's atoms in the order of their arrival: the rank then reads a cell's sort
+// keys contiguously and its own atom's fields coalesced, instead of through the
+// order (128 uneven replicas that rebuild together 343 -> 339 us per step, 1M
+// beads 193.4 -> 192.9).
 __global__ void __launch_bounds__(256) k_scatter(REBUILD_ARGS) {
     REBUILD_LOOP {
         REBUILD_PROLOGUE
         if (i < d.natoms) {
-            const int dst = d.cell_start[d.cell_of[i]] + d.rank[i];
-            d.order[dst] = i;
-            d.tmp_pos[i] = d.pos[i];
-            d.tmp_vel[i] = d.vel[i];
-            d.tmp_img[i] = d.img[i];
+            const int key = d.cell_of[i], dst = d.cell_start[key] + d.rank[i];
+            d.order[dst] = key;
+            d.order2[dst] = d.sortx[i];
+            d.tmp_pos[dst] = d.pos[i];
+            d.tmp_vel[dst] = d.vel[i];
+            d.tmp_img[dst] = d.img[i];
         }
         // the tile's share of the cell counts, cleared for the next rebuild
         const int nkeys = 1 << (3 * st->cbits), per = (nkeys + d.ntiles - 1) / d.ntiles;
@@ -853,23 +859,20 @@ __global__ void __launch_bounds__(256) k_rank(REBUILD_ARGS) {
     REBUILD_LOOP {
         REBUILD_PROLOGUE
         if (i < d.natoms) {
-            const int src = d.order[i];
-            const int key = d.cell_of[src];
+            const int key = d.order[i];
             const int s = d.cell_start[key], e = d.cell_start[key + 1];
-            const int g = d.tmp_img[src].w;
-            const int rx = d.sortx[src];
+            const int4 im = d.tmp_img[i];
+            const int rx = d.order2[i];
             int r = 0;
             for (int q = s; q < e; q++) {
-                const int o = d.order[q];
-                const int ro = d.sortx[o];
-                r += (ro < rx) || (ro == rx && d.tmp_img[o].w < g);
+                const int ro = d.order2[q];
+                r += (ro < rx) || (ro == rx && d.tmp_img[q].w < im.w);
             }
             const int dst = s + r;
-            const float4 p = d.tmp_pos[src];
-            const int4 im = d.tmp_img[src];
+            const float4 p = d.tmp_pos[i];
             d.pos[dst] = p;
             d.pos_ref[dst] = p;
-            d.vel[dst] = d.tmp_vel[src];
+            d.vel[dst] = d.tmp_vel[i];
             d.img[dst] = im;
             d.gid[dst] = im.w;
             d.slot_of[im.w] = dst;
