@@ -2622,10 +2622,20 @@ __global__ void __launch_bounds__(kBndThreads) k_boundary(const RepDesc* __restr
     const RepDesc& d = descs[reps[blockIdx.x]];
     RepState* const gst = d.st;
     RepState* const st = (RepState*)s_state;
-    if (mode == BND_STEP && d.ensemble == 0 && !gst->want_obs) {  // uniform
+    // The flags that the branches below go by are read by every wave ahead of the
+    // barrier, and written (by thread 0: start_step sets all of them for the next
+    // step) only behind it, so they are uniform over the workgroup.
+    const int active = __builtin_amdgcn_readfirstlane(gst->active);
+    const int ready = __builtin_amdgcn_readfirstlane(gst->pre_ready);
+    const int want_obs = __builtin_amdgcn_readfirstlane(gst->want_obs);
+    const bool quiet = mode == BND_STEP && d.ensemble == 0 && !want_obs;
+    if (!quiet && threadIdx.x < kStWords) ((int*)s_state)[threadIdx.x] = gview((const int*)gst)[threadIdx.x];
+    __syncthreads();
+    if (mode == BND_START ? (!active || ready) : (mode == BND_STEP && !active)) return;
+    if (quiet) {
         // a Langevin step that records nothing reduced no partials (k_force): the
         // step count and the next step's target only
-        if (threadIdx.x == 0 && gst->active) {
+        if (threadIdx.x == 0) {
             const int64_t cur = gst->step + 1, stop = gst->stop;
             const int err = gst->err;
             gst->v_pending = 1.0f;
@@ -2641,9 +2651,6 @@ __global__ void __launch_bounds__(kBndThreads) k_boundary(const RepDesc* __restr
         }
         return;
     }
-    if (threadIdx.x < kStWords) ((int*)s_state)[threadIdx.x] = gview((const int*)gst)[threadIdx.x];
-    __syncthreads();
-    if (mode == BND_START ? !(st->active && !st->pre_ready) : mode == BND_STEP && !st->active) return;  // uniform
     if (mode == BND_START) {
         if (threadIdx.x == 0) {
             start_step(d, st, st->step + 1);
