@@ -1492,11 +1492,13 @@ k_build(REBUILD_ARGS) {
                     // list: the distance along y and z to the row's cells leaves
                     // at most sqrt(rb2 - dy^2 - dz^2) along x, and the coarse x
                     // difference is within one unit of the true one.  A row with
-                    // nothing left is skipped whole.
+                    // nothing left is skipped whole.  In a box of three cells an
+                    // atom on a cell bound (its float cell coordinate one low) has
+                    // an outer cell's far side in reach too: no limit along x there.
                     const int dyb = (iy == 1) ? 0 : yb[iy >> 1], dzb = (iz == 1) ? 0 : zb[iz >> 1];
                     const int rem = rb2 - dyb * dyb - dzb * dzb;
                     if (rem < 0) continue;
-                    const int xr = (int)ceilf(sqrtf((float)rem)) + 2;
+                    const int xr = nx > 3 ? (int)ceilf(sqrtf((float)rem)) + 2 : 65536;
                     const int wb = (wmod(rz + iz - 1 - sz, ez_) * ey_ + wmod(ry + iy - 1 - sy, ey_)) * ex_;
                     const int ua = s_wmap[wb + w0], ub = s_wmap[wb + w1], uc = s_wmap[wb + w2];
                     if (ua >= nu || ub >= nu || uc >= nu) {  // every neighbor cell was marked; guard regardless
