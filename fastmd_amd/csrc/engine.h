@@ -4,6 +4,7 @@
 
 #include <cstdint>
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -196,7 +197,8 @@ class Engine {
     Launch launch_of(const Batch& b, hipStream_t s) const;
     int32_t read_state(Replica& r, RepState& s);
     // Pinned host memory of at least n bytes (null: none to be had), kept by the
-    // engine and grown to at most 2 kReadBytes.
+    // engine and grown to at most 2 kReadBytes; asked for and used under read_mu_
+    // (reads of one engine may come from several threads).
     char* pinned(size_t n);
     void reserve_read(int natoms);
     // Launches `read` for each range of at most kReadAtoms global ids into one of
@@ -211,6 +213,7 @@ class Engine {
     hipStream_t stream_ = nullptr;
     hipStream_t side_ = nullptr;  // system creation beside the main stream's launches
     hipStream_t aux_ = nullptr;   // a step's list rebuilds beside its force pass
+    std::mutex read_mu_;          // of the readback buffer and its events
     char* pin_ = nullptr;         // readback buffer (pinned)
     size_t pin_bytes_ = 0;
     hipEvent_t ev_read_[2] = {nullptr, nullptr};

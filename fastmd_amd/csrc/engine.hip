@@ -967,6 +967,7 @@ static size_t range_bytes(int natoms, size_t per_atom) {
 // With the system, so that its first readback does not pay for the buffer; a
 // failure is reported by the readback that needs it.
 void Engine::reserve_read(int natoms) {
+    std::lock_guard<std::mutex> g(read_mu_);
     if (!pinned(range_bytes(natoms, 40) * (natoms > kReadAtoms ? 2 : 1) + 4096)) err_.clear();
 }
 
@@ -974,6 +975,7 @@ template <class Read, class Take>
 int32_t Engine::read_ranges(int natoms, size_t per_atom, hipStream_t s, Read&& read, Take&& take) {
     const int nr = (natoms + kReadAtoms - 1) / kReadAtoms;
     const size_t half = range_bytes(natoms, per_atom);
+    std::lock_guard<std::mutex> g(read_mu_);
     char* buf = pinned(nr > 1 ? 2 * half : half);
     if (!buf) return FMD_ERR_NOMEM;
     int32_t rc = FMD_OK;
@@ -1226,6 +1228,7 @@ int32_t Engine::compute_forces(int32_t sys, uint32_t terms, float* f4, double* v
     const size_t head = (sizeof(RepState) + 255) / 256 * 256;
     int32_t rc;
     if (f4 && r->natoms <= kReadAtoms) {  // the state with the forces: one wait
+        std::lock_guard<std::mutex> g(read_mu_);
         char* b = pinned(head + (size_t)r->natoms * 16);
         rc = b ? FMD_OK : FMD_ERR_NOMEM;
         if (!rc) {
