@@ -759,63 +759,121 @@ __global__ void __launch_bounds__(256) k_bin(REBUILD_ARGS) {
 }
 
 // Exclusive scan of the cell counts (k_scatter clears them for the next
-// rebuild).  Workgroup (replica, y) of 1024 threads scans kScanKeys keys, four
-// consecutive ones a thread, from the sum of all the counts before them, which
-// it forms itself, instead of one workgroup that carries the sum through all keys
-// (115 us for the 262,144 keys of 1M beads).  1M beads: 200.1 -> 195.5 us per step.
+// rebuild).  Workgroup (replica, y) of 1024 threads scans a run of keys in
+// passes of kScanKeys, four consecutive ones a thread, from the sum of all the
+// counts before it.  With up to kScanBlocks workgroups it forms that sum itself
+// (1M beads, 262,144 keys: 195.5 us per step; one workgroup that carries the sum
+// through all keys 200.1).  What is read so grows with the square of the keys,
+// so for boxes of more keys the runs' totals are formed first (k_scan_totals,
+// into the replica's `order`, which the sort writes later) and each workgroup
+// sums those.  A list rebuild of 4,000 beads by one workgroup / by 64 / with
+// totals: 2,097,152 keys 910 / 317 / 132 us, 16.8M 6.2 / 1.6 / 0.27 ms.
 constexpr int kScanKeys = 4096;
+constexpr int kScanBlocks = 64;   // workgroups a replica without totals
+constexpr int kScanTotals = 256;  // and with: `order` holds at least a group's slots
+static_assert(kScanTotals <= kGroupSlots, "a replica has at least a group of slots");
+__device__ inline int scan_run(int nkeys) {  // keys of one workgroup
+    const int pass = (int)gridDim.y * kScanKeys;
+    return (nkeys + pass - 1) / pass * kScanKeys;
+}
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+__global__ void __launch_bounds__(1024) k_scan_totals(const RepDesc* __restrict__ descs,
+                                                      const int* __restrict__ reps, int nr, int always) {
+    __shared__ int wsum[16];
+    const RepDesc& d = descs[reps[blockIdx.x]];
+    const RepState* st = d.st;
+    if (!always && !(st->active && st->rebuild)) return;
+    const int nkeys = 1 << (3 * st->cbits), run = scan_run(nkeys), k0 = blockIdx.y * run;
+    if (k0 >= nkeys || nkeys < 4) return;  // 1 key, or a multiple of 4
+    const FMD_GLOBAL int* cnt = gview(d.cell_cnt);
+    const int end = min(k0 + run, nkeys);
+    int sum = 0;
+#pragma unroll 4
+    for (int k = k0 + 4 * threadIdx.x; k < end; k += kScanKeys) {
+        const i32x4 v = *(const FMD_GLOBAL i32x4*)(cnt + k);
+        sum += v.x + v.y + v.z + v.w;
+    }
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) sum += __shfl_xor(sum, o, 64);
+    if (lane_id() == 0) wsum[threadIdx.x >> 6] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int total = 0;
+#pragma unroll
+        for (int w = 0; w < 16; w++) total += wsum[w];
+        gmut(d.order)[blockIdx.y] = total;
+    }
+}
+template <bool TOTALS>
 __global__ void __launch_bounds__(1024) k_scan(const RepDesc* __restrict__ descs,
                                                const int* __restrict__ reps, int nr, int always) {
     __shared__ int wsum[16], wbase[16];
     const RepDesc& d = descs[reps[blockIdx.x]];
     RepState* st = d.st;
     if (!always && !(st->active && st->rebuild)) return;
-    const int nkeys = 1 << (3 * st->cbits);
-    const int k0 = blockIdx.y * kScanKeys;
+    const int nkeys = 1 << (3 * st->cbits), run = scan_run(nkeys), k0 = blockIdx.y * run;
     if (k0 >= nkeys) return;
-    const int lane = lane_id(), wv = threadIdx.x >> 6, c0 = k0 + 4 * threadIdx.x;
+    const int lane = lane_id(), wv = threadIdx.x >> 6, end = min(k0 + run, nkeys);
     const FMD_GLOBAL int* cnt = gview(d.cell_cnt);
-    typedef int i32x4 __attribute__((ext_vector_type(4)));
-    int before = 0;  // k0 is a multiple of kScanKeys: whole 16-byte loads
+    int before = 0;
+    if (TOTALS) {
+        if (threadIdx.x < blockIdx.y) before = gview(d.order)[threadIdx.x];
+    } else {
 #pragma unroll 4
-    for (int k = 4 * threadIdx.x; k < k0; k += kScanKeys) {
-        const i32x4 v = *(const FMD_GLOBAL i32x4*)(cnt + k);
-        before += v.x + v.y + v.z + v.w;
-    }
-    int v[4] = {0, 0, 0, 0};
-    if (c0 + 3 < nkeys) {
-        const i32x4 q = *(const FMD_GLOBAL i32x4*)(cnt + c0);
-        v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
-    } else {
-#pragma unroll
-        for (int k = 0; k < 4; k++)
-            if (c0 + k < nkeys) v[k] = cnt[c0 + k];
-    }
-    const int local = v[0] + v[1] + v[2] + v[3];
-    int x = local;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-        before += __shfl_xor(before, o, 64);
-    }
-    if (lane == 63) wsum[wv] = x;
-    if (lane == 0) wbase[wv] = before;
-    __syncthreads();
-    int run = x - local;
-#pragma unroll
-    for (int w = 0; w < 16; w++) run += wbase[w] + (w < wv ? wsum[w] : 0);
-    FMD_GLOBAL int* out = gmut(d.cell_start) + c0;
-    if (c0 + 3 < nkeys) {
-        *(FMD_GLOBAL i32x4*)out = i32x4{run, run + v[0], run + v[0] + v[1], run + v[0] + v[1] + v[2]};
-    } else {
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            if (c0 + k < nkeys) out[k] = run;
-            run += v[k];
+        for (int k = 4 * threadIdx.x; k < k0; k += kScanKeys) {  // k0 is a multiple of kScanKeys
+            const i32x4 v = *(const FMD_GLOBAL i32x4*)(cnt + k);
+            before += v.x + v.y + v.z + v.w;
         }
     }
-    if (c0 < nkeys && c0 + 4 >= nkeys) gmut(d.cell_start)[nkeys] = d.natoms;
+    int v[4];
+    auto load = [&](int p0) __attribute__((always_inline)) {
+        const int c0 = p0 + 4 * threadIdx.x;
+        if (c0 + 3 < nkeys) {
+            const i32x4 q = *(const FMD_GLOBAL i32x4*)(cnt + c0);
+            v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; k++) v[k] = c0 + k < nkeys ? cnt[c0 + k] : 0;
+        }
+    };
+    load(k0);
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) before += __shfl_xor(before, o, 64);
+    if (lane == 0) wbase[wv] = before;
+    int carry = 0;  // counts of this workgroup's earlier passes
+    for (int p0 = k0; p0 < end; p0 += kScanKeys) {
+        const int c0 = p0 + 4 * threadIdx.x;
+        const int local = v[0] + v[1] + v[2] + v[3];
+        int x = local;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(x, o, 64);
+            if (lane >= o) x += y;
+        }
+        if (lane == 63) wsum[wv] = x;
+        __syncthreads();
+        int at = carry + x - local;
+#pragma unroll
+        for (int w = 0; w < 16; w++) {
+            const int ws = wsum[w];
+            at += wbase[w] + (w < wv ? ws : 0);
+            carry += ws;
+        }
+        FMD_GLOBAL int* out = gmut(d.cell_start) + c0;
+        if (c0 + 3 < nkeys) {
+            *(FMD_GLOBAL i32x4*)out = i32x4{at, at + v[0], at + v[0] + v[1], at + v[0] + v[1] + v[2]};
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                if (c0 + k < nkeys) out[k] = at;
+                at += v[k];
+            }
+        }
+        if (c0 < nkeys && c0 + 4 >= nkeys) gmut(d.cell_start)[nkeys] = d.natoms;
+        if (p0 + kScanKeys >= end) break;
+        load(p0 + kScanKeys);
+        __syncthreads();  // wsum is rewritten by the next pass
+    }
 }
 
 // Atoms, their keys (order) and sort keys (order2) stored in cell order, a
@@ -2822,6 +2880,23 @@ void launch_control(const Launch& l, int op, int64_t arg) {
 static constexpr int kMaxBlock = kMaxBlockK;
 static inline int valid_block(int b) { return (b == 64 || b == 128 || b == 256) ? b : kMaxBlock; }
 
+// The workgroups of the scan: one a pass of keys of the largest replica, as far
+// as their limits and kScanGrid for the whole batch go.  Those of replicas that
+// do not rebuild, or have fewer keys, return at once, but they are launched in
+// every step (1,023 small replicas and one of 2,097,152 keys: 680 us per step
+// with a workgroup a pass for each replica, 145 with two a replica).
+static constexpr int kScanGrid = 2048;
+static void launch_scan(const Launch& l, int always) {
+    const int passes = cdiv(l.max_keys, kScanKeys), share = max(1, kScanGrid / l.nr);
+    const bool totals = min(passes, share) > kScanBlocks;
+    const dim3 g(l.nr, min(min(passes, share), totals ? kScanTotals : kScanBlocks));
+    if (totals) {
+        k_scan_totals<<<g, 1024, 0, l.stream>>>(l.descs, l.reps, l.nr, always);
+        k_scan<true><<<g, 1024, 0, l.stream>>>(l.descs, l.reps, l.nr, always);
+    } else {
+        k_scan<false><<<g, 1024, 0, l.stream>>>(l.descs, l.reps, l.nr, always);
+    }
+}
 void launch_rebuild(const Launch& l, int always, int build) {
     if (l.ntl <= 0) return;
     // a step's rebuild tile list is k_decide's; otherwise list the tiles here
@@ -2829,7 +2904,7 @@ void launch_rebuild(const Launch& l, int always, int build) {
     int g = cdiv(l.ntl, 4);
     if (g > kStrideBlocks) g = kStrideBlocks;
     k_bin<<<g, 256, 0, l.stream>>>(l.descs, l.tiles, l.rlist, l.nrt);
-    k_scan<<<dim3(l.nr, cdiv(l.max_keys, kScanKeys)), 1024, 0, l.stream>>>(l.descs, l.reps, l.nr, always);
+    launch_scan(l, always);
     k_scatter<<<g, 256, 0, l.stream>>>(l.descs, l.tiles, l.rlist, l.nrt);
     k_rank<<<g, 256, 0, l.stream>>>(l.descs, l.tiles, l.rlist, l.nrt);
     if (build) launch_build(l);
