@@ -955,7 +955,10 @@ char* Engine::pinned(size_t n) {
     pin_ = nullptr;
     pin_bytes_ = 0;
     void* p = nullptr;
-    if (hip_check(hipHostMalloc(&p, want, hipHostMallocDefault), "hipHostMalloc")) return nullptr;
+    if (hip_check(hipHostMalloc(&p, want, hipHostMallocDefault), "hipHostMalloc")) {
+        (void)hipGetLastError();  // reported here, not by the next launch's check
+        return nullptr;
+    }
     pin_ = (char*)p;
     pin_bytes_ = want;
     return pin_;
