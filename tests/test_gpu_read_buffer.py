@@ -67,7 +67,7 @@ try:
     e.state(s)
     raise SystemExit("the readback did not report it")
 except fmd.FmdError as x:
-    assert x.code == fmd.ERR_NOMEM, x
+    assert x.code == fmd.api.ERR_NOMEM, x
 e.step(s, 5)
 p, v, im = e.state(s)         # there is memory again
 assert np.isfinite(p).all() and e.steps_done(s) == 10
