@@ -216,6 +216,7 @@ class Engine {
     std::mutex read_mu_;          // of the readback buffer and its events
     char* pin_ = nullptr;         // readback buffer (pinned)
     size_t pin_bytes_ = 0;
+    std::vector<char*> pin_old_;  // smaller ones it took the place of, freed with the deferred blocks
     hipEvent_t ev_read_[2] = {nullptr, nullptr};
     hipEvent_t ev_fork_ = nullptr, ev_sorted_ = nullptr, ev_join_ = nullptr;
     double* scratch_ = nullptr;   // this device's scratch array (device address), or null

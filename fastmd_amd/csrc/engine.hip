@@ -87,6 +87,7 @@ Engine::~Engine() {
     if (side_) (void)hipStreamDestroy(side_);
     if (aux_) (void)hipStreamDestroy(aux_);
     if (pin_) (void)hipHostFree(pin_);
+    for (char* p : pin_old_) (void)hipHostFree(p);
     for (auto& ev : ev_read_)
         if (ev) (void)hipEventDestroy(ev);
     if (ev_fork_) (void)hipEventDestroy(ev_fork_);
@@ -144,6 +145,11 @@ void Engine::release_block(void* p, size_t bytes) {
 
 void Engine::flush_deferred() {
     defer_free_ = false;
+    {
+        std::lock_guard<std::mutex> g(read_mu_);
+        for (char* p : pin_old_) (void)hipHostFree(p);
+        pin_old_.clear();
+    }
     flush_cache(std::min<uint64_t>(budget_ / 8, 8ull << 30));
 }
 
@@ -951,14 +957,14 @@ char* Engine::pinned(size_t n) {
     size_t want = 256 << 10;
     while (want < n) want *= 2;
     want = std::min(want, std::max(n, 2 * kReadBytes));
-    if (pin_) (void)hipHostFree(pin_);
-    pin_ = nullptr;
-    pin_bytes_ = 0;
     void* p = nullptr;
     if (hip_check(hipHostMalloc(&p, want, hipHostMallocDefault), "hipHostMalloc")) {
         (void)hipGetLastError();  // reported here, not by the next launch's check
         return nullptr;
     }
+    // hipHostFree waits for the device: not while a launch runs
+    if (pin_ && defer_free_) pin_old_.push_back(pin_);
+    else if (pin_) (void)hipHostFree(pin_);
     pin_ = (char*)p;
     pin_bytes_ = want;
     return pin_;

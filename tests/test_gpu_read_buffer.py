@@ -1,6 +1,8 @@
-"""The engine's pinned readback buffer where the HIP runtime cannot give it.  A
-process of its own loads a shim ahead of the library whose hipHostMalloc can be
-told to ask for more than there is, so that the call fails in the runtime."""
+"""The engine's pinned readback buffer: where the HIP runtime cannot give it, and
+where it grows while a server's launch runs.  A process of its own loads a shim
+ahead of the library whose hipHostMalloc can be told to ask for more than there
+is, so that the call fails in the runtime, and which counts the frees of pinned
+memory between a graph launch and the wait for its stream."""
 import os
 import subprocess
 import sys
@@ -17,10 +19,28 @@ SHIM = r"""
 static void* runtime(const char* name) {
     return dlsym(dlopen("libamdhip64.so.7", RTLD_LAZY | RTLD_NOLOAD), name);
 }
+int allocs = 0;
 int fail_allocs = 0;  /* allocations still to fail */
 int hipHostMalloc(void** p, size_t n, unsigned flags) {
     int (*real)(void**, size_t, unsigned) = (int (*)(void**, size_t, unsigned))runtime("hipHostMalloc");
+    allocs++;
     return real(p, fail_allocs > 0 && fail_allocs-- ? (size_t)1 << 60 : n, flags);
+}
+static void* volatile launched = 0;  /* the stream of a graph launch not waited for yet */
+int frees = 0, frees_in_launch = 0;
+int hipGraphLaunch(void* graph, void* stream) {
+    launched = stream;
+    return ((int (*)(void*, void*))runtime("hipGraphLaunch"))(graph, stream);
+}
+int hipStreamSynchronize(void* stream) {
+    int rc = ((int (*)(void*))runtime("hipStreamSynchronize"))(stream);
+    if (stream == launched) launched = 0;
+    return rc;
+}
+int hipHostFree(void* p) {
+    frees++;
+    if (launched) frees_in_launch++;
+    return ((int (*)(void*))runtime("hipHostFree"))(p);
 }
 """
 
@@ -72,5 +92,29 @@ e.step(s, 5)
 p, v, im = e.state(s)         # there is memory again
 assert np.isfinite(p).all() and e.steps_done(s) == 10
 e.close()
+print("ok")
+""")
+
+
+def test_growth_beside_a_launch_frees_nothing_until_it_ends(tmp_path):
+    _run(tmp_path, r"""
+import time
+s = fmd.Server(0)
+a = s.submit(desc(300), 60000)
+while s.stats()["graph_launches"] < 20:
+    time.sleep(0.002)
+before = var("allocs").value
+jobs = [s.submit(desc(n, n), 40) for n in (9000, 20000, 60000)]
+while any(s.poll(j) not in (2, 3) for j in jobs):
+    time.sleep(0.002)
+running = s.poll(a) == 1
+s.drain()
+for j, n in zip([a] + jobs, (300, 9000, 20000, 60000)):
+    r = s.result(j, state=True)
+    assert r["status"] == 0 and np.isfinite(r["pos4"]).all() and len(r["pos4"]) == n
+print("grown", var("allocs").value - before, "freed", var("frees").value, "beside a launch", var("frees_in_launch").value)
+assert running and var("allocs").value > before and var("frees").value > 0
+assert var("frees_in_launch").value == 0
+s.close()
 print("ok")
 """)
