@@ -54,6 +54,7 @@ struct Replica {
     int id = -1;
     int natoms = 0, nslots = 0, ntiles = 0, cls = 0;
     int ensemble = 0;
+    bool sums_always = false;  // every step forms its sums: a Nose-Hoover chain, or a record or sample a step
     RepDesc desc{};         // host copy of the device descriptor
     RepState* st = nullptr; // device
     void* block = nullptr;  // the replica's device arrays, carved from one block
@@ -74,7 +75,7 @@ struct Batch {
     int* d_nrt = nullptr;     // its length
     Tile* d_chunks = nullptr; // (replica, chunk of kChunkTiles tiles) list
     int nch = 0, max_chunks = 0, max_keys = 0;
-    bool any_nh = false;      // a replica with a Nose-Hoover chain
+    bool sums_always = false; // a replica whose every step forms its sums
     bool any_tab = false;     // a replica with tabulated pairs
     int4* d_status = nullptr; // per replica (err, active, step lo, step hi), d_reps order
     int* d_phase = nullptr;   // per replica, steps since its last list build (d_reps order)

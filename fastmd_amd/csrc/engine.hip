@@ -337,6 +337,7 @@ int32_t Engine::create_impl(const fmd_system_desc* d, int32_t* sys, int kmult, b
     r.natoms = S.natoms; r.nslots = S.nslots; r.ntiles = S.ntiles;
     r.cls = size_class(S.natoms);
     r.ensemble = d->ensemble;
+    r.sums_always = d->ensemble != FMD_LANGEVIN || d->thermo_freq == 1 || d->stress_freq == 1;
     r.thermo_cap = S.thermo_cap;
     RepDesc& D = r.desc;
     std::memset(&D, 0, sizeof(D));
@@ -739,7 +740,7 @@ Batch* Engine::batch_for(const std::vector<int>& ids_in) {
     b->wgsort = true;
     for (int id : ord) {
         b->max_chunks = std::max(b->max_chunks, reps_[id]->desc.nchunks);
-        b->any_nh = b->any_nh || reps_[id]->ensemble != FMD_LANGEVIN;
+        b->sums_always = b->sums_always || reps_[id]->sums_always;
         b->any_tab = b->any_tab || reps_[id]->desc.ntables > 0;
         b->max_keys = std::max(b->max_keys, reps_[id]->desc.ncell_cap);
         b->max_atoms = std::max(b->max_atoms, reps_[id]->natoms);
@@ -792,7 +793,7 @@ void Engine::free_batch(Batch* b) {
 
 Launch Engine::launch_of(const Batch& b) const { return launch_of(b, stream_); }
 Launch Engine::launch_of(const Batch& b, hipStream_t s) const {
-    return Launch{d_descs_, b.d_tiles, b.ntl, b.d_reps, b.nr, b.d_rep_t0, b.d_rlist, b.d_nrt, b.d_chunks, b.nch, b.max_chunks, b.max_keys, b.any_tab, b.any_nh, s};
+    return Launch{d_descs_, b.d_tiles, b.ntl, b.d_reps, b.nr, b.d_rep_t0, b.d_rlist, b.d_nrt, b.d_chunks, b.nch, b.max_chunks, b.max_keys, b.any_tab, b.sums_always, s};
 }
 
 // Whether the batch's steps build lists beside the force pass: with enough
@@ -1457,6 +1458,12 @@ int32_t Engine::resume(const void* buf, uint64_t size, int32_t* sys) {
     r.id = id;
     r.natoms = h.natoms; r.nslots = h.nslots; r.ntiles = h.ntiles; r.cls = h.cls;
     r.ensemble = h.ensemble; r.thermo_cap = h.thermo_cap;
+    {
+        RepState s{};
+        const uintptr_t o = (uintptr_t)h.desc.st - 1;
+        if (o + sizeof(s) <= h.used) std::memcpy(&s, (const char*)buf + sizeof(SnapHeader) + o, sizeof(s));
+        r.sums_always = h.ensemble != FMD_LANGEVIN || s.thermo_freq == 1 || s.stress_freq == 1;
+    }
     r.steps_done = h.steps_done; r.thermo_read = h.thermo_read;
     r.block = base; r.block_bytes = got; r.block_used = h.used; r.bytes = charge_bytes(h.used);
     r.desc = h.desc;

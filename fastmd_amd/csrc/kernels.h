@@ -21,7 +21,7 @@ struct Launch {
     int max_chunks;        // of one replica
     int max_keys;          // cell keys, the largest capacity of one replica
     bool any_tab;          // a replica with tabulated pairs
-    bool any_nh;           // a replica with a Nose-Hoover chain (partials on every step)
+    bool sums_always;      // a replica whose every step forms its sums (a chain, or a record or sample a step)
     hipStream_t stream;
 };
 

@@ -2664,10 +2664,11 @@ __device__ int boundary_tail(const RepDesc& d, RepState* st, int mode, const dou
 // batch of replicas of at most kFusedChunks chunks) the first reduction level
 // is done here too, chunk after chunk, instead of by a k_chunk launch: worth the
 // launch for one chunk, or for several where most steps sum nothing (no chain
-// reads the kinetic energy), but two chunks one after the other take longer
-// than the launch (30,000 beads NVT 50.4 us per step against 49.2).  Together
-// per step: 2,000 beads 31.5 -> 28.6 us, 30,000 44.5 -> 41.7, NPT 120,000
-// 72.1 -> 69.1, 48 small replicas 70.1 -> 63.2.
+// reads the kinetic energy, no record or sample on every step), but two chunks
+// one after the other take longer than the launch (30,000 beads NVT 50.4 us per
+// step against 49.2; four with a record a step, 60,000 beads, 49.6 against
+// 45.1).  Together per step: 2,000 beads 31.5 -> 28.6 us, 30,000 44.5 -> 41.7,
+// NPT 120,000 72.1 -> 69.1, 48 small replicas 70.1 -> 63.2.
 template <bool FUSED>
 __global__ void __launch_bounds__(kBndThreads) k_boundary(const RepDesc* __restrict__ descs,
                                                           const int* __restrict__ reps, int nr, int mode) {
@@ -2955,7 +2956,7 @@ void launch_force_listed(const Launch& l, int kick, int mode) {
 }
 void launch_boundary(const Launch& l, int mode) {
     if (l.nr <= 0) return;
-    if (mode == BND_START || l.max_chunks <= (l.any_nh ? 1 : kFusedChunks)) {
+    if (mode == BND_START || l.max_chunks <= (l.sums_always ? 1 : kFusedChunks)) {
         k_boundary<true><<<l.nr, kBndThreads, 0, l.stream>>>(l.descs, l.reps, l.nr, mode);
         return;
     }

@@ -59,3 +59,24 @@ def test_batch_with_observed_and_unobserved_steps(fmd, engine, freq):
         engine.remove(a)
     for s in sids:
         engine.remove(s)
+
+
+@pytest.mark.parametrize("n", [16385, 40000, 65000])
+def test_sums_of_every_step_and_of_the_last(fmd, engine, n):
+    """Langevin replicas of two to four chunks: observed at every step (the chunks
+    summed by a launch of their own) and at the last only (in the boundary's
+    workgroup), the same state and the same last record, resumed ones included."""
+    descs = [_desc(fmd, n, 0, 1, 0), _desc(fmd, n, 0, STEPS, 0)]
+    sids = [engine.add(d) for d in descs]
+    for s in sids:
+        engine.step(s, STEPS - 4)
+    sids.append(engine.resume(engine.snapshot(sids[0])))
+    for s in sids:
+        engine.step(s, 4)
+    last = [engine.drain_thermo(s)[0][-1] for s in sids]
+    assert last[0] == last[1] == last[2] and last[0]["step"] == STEPS
+    for s in sids[1:]:
+        for u, w in zip(engine.state(sids[0]), engine.state(s)):
+            assert np.array_equal(u, w)
+    for s in sids:
+        engine.remove(s)
