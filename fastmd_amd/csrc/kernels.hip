@@ -804,7 +804,10 @@ __global__ void __launch_bounds__(1024) k_scan_totals(const RepDesc* __restrict_
         gmut(d.order)[blockIdx.y] = total;
     }
 }
-template <bool TOTALS>
+// ONE: no workgroup has more than one pass.  At most 40 VGPRs: in the forked step
+// a workgroup waits for its 16 waves' registers to come free beside the force
+// pass (256 replicas: 33 us with 33 VGPRs, 167 with 50).
+template <bool ONE, bool TOTALS>
 __global__ void __launch_bounds__(1024) k_scan(const RepDesc* __restrict__ descs,
                                                const int* __restrict__ reps, int nr, int always) {
     __shared__ int wsum[16], wbase[16];
@@ -825,9 +828,8 @@ __global__ void __launch_bounds__(1024) k_scan(const RepDesc* __restrict__ descs
             before += v.x + v.y + v.z + v.w;
         }
     }
-    int v[4];
-    auto load = [&](int p0) __attribute__((always_inline)) {
-        const int c0 = p0 + 4 * threadIdx.x;
+    int c0 = k0 + 4 * threadIdx.x, v[4];
+    auto load = [&]() __attribute__((always_inline)) {
         if (c0 + 3 < nkeys) {
             const i32x4 q = *(const FMD_GLOBAL i32x4*)(cnt + c0);
             v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
@@ -836,13 +838,17 @@ __global__ void __launch_bounds__(1024) k_scan(const RepDesc* __restrict__ descs
             for (int k = 0; k < 4; k++) v[k] = c0 + k < nkeys ? cnt[c0 + k] : 0;
         }
     };
-    load(k0);
+    load();
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) before += __shfl_xor(before, o, 64);
     if (lane == 0) wbase[wv] = before;
-    int carry = 0;  // counts of this workgroup's earlier passes
-    for (int p0 = k0; p0 < end; p0 += kScanKeys) {
-        const int c0 = p0 + 4 * threadIdx.x;
+    int carry = 0;  // the counts before this pass, less those in wbase if there is one pass only
+    if (!ONE) {
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < 16; w++) carry += wbase[w];
+    }
+    for (int p0 = k0;; p0 += kScanKeys) {
         const int local = v[0] + v[1] + v[2] + v[3];
         int x = local;
 #pragma unroll
@@ -856,8 +862,8 @@ __global__ void __launch_bounds__(1024) k_scan(const RepDesc* __restrict__ descs
 #pragma unroll
         for (int w = 0; w < 16; w++) {
             const int ws = wsum[w];
-            at += wbase[w] + (w < wv ? ws : 0);
-            carry += ws;
+            at += (ONE ? wbase[w] : 0) + (w < wv ? ws : 0);
+            if (!ONE) carry += ws;
         }
         FMD_GLOBAL int* out = gmut(d.cell_start) + c0;
         if (c0 + 3 < nkeys) {
@@ -870,8 +876,9 @@ __global__ void __launch_bounds__(1024) k_scan(const RepDesc* __restrict__ descs
             }
         }
         if (c0 < nkeys && c0 + 4 >= nkeys) gmut(d.cell_start)[nkeys] = d.natoms;
-        if (p0 + kScanKeys >= end) break;
-        load(p0 + kScanKeys);
+        if (ONE || p0 + kScanKeys >= end) break;
+        c0 += kScanKeys;
+        load();
         __syncthreads();  // wsum is rewritten by the next pass
     }
 }
@@ -2893,9 +2900,11 @@ static void launch_scan(const Launch& l, int always) {
     const dim3 g(l.nr, min(min(passes, share), totals ? kScanTotals : kScanBlocks));
     if (totals) {
         k_scan_totals<<<g, 1024, 0, l.stream>>>(l.descs, l.reps, l.nr, always);
-        k_scan<true><<<g, 1024, 0, l.stream>>>(l.descs, l.reps, l.nr, always);
+        k_scan<false, true><<<g, 1024, 0, l.stream>>>(l.descs, l.reps, l.nr, always);
+    } else if (passes <= (int)g.y) {
+        k_scan<true, false><<<g, 1024, 0, l.stream>>>(l.descs, l.reps, l.nr, always);
     } else {
-        k_scan<false><<<g, 1024, 0, l.stream>>>(l.descs, l.reps, l.nr, always);
+        k_scan<false, false><<<g, 1024, 0, l.stream>>>(l.descs, l.reps, l.nr, always);
     }
 }
 void launch_rebuild(const Launch& l, int always, int build) {
