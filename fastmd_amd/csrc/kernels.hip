@@ -1224,7 +1224,11 @@ k_build(REBUILD_ARGS) {
             const double rin = rc * sqrt(1.0 - band) - 1.7321 - 0.01, rout = rb + 1.7321 + 0.01;
             clo = __builtin_amdgcn_readfirstlane(rin > 0.0 ? (int)floor(rin * rin) : 0);
             chi = __builtin_amdgcn_readfirstlane((int)ceil(rout * rout));
-            rb2 = __builtin_amdgcn_readfirstlane((int)fmin(ceil(rb * rb) + 1.0, 2147483647.0));
+            // In a box of three cells an atom on a cell bound (its float cell
+            // coordinate one low) has an outer cell's far side in reach along x:
+            // there the rows are not cut short (the pair's y and z distances are
+            // next to nothing, so more than two cells are left of this along x).
+            rb2 = __builtin_amdgcn_readfirstlane(nx > 3 ? (int)fmin(ceil(rb * rb) + 1.0, 2147483647.0) : INT_MAX);
         }
         int nu = 0, nstage = 0;
         if (staged) {
@@ -1557,13 +1561,11 @@ k_build(REBUILD_ARGS) {
                     // list: the distance along y and z to the row's cells leaves
                     // at most sqrt(rb2 - dy^2 - dz^2) along x, and the coarse x
                     // difference is within one unit of the true one.  A row with
-                    // nothing left is skipped whole.  In a box of three cells an
-                    // atom on a cell bound (its float cell coordinate one low) has
-                    // an outer cell's far side in reach too: no limit along x there.
+                    // nothing left is skipped whole.
                     const int dyb = (iy == 1) ? 0 : yb[iy >> 1], dzb = (iz == 1) ? 0 : zb[iz >> 1];
                     const int rem = rb2 - dyb * dyb - dzb * dzb;
                     if (rem < 0) continue;
-                    const int xr = nx > 3 ? (int)ceilf(sqrtf((float)rem)) + 2 : 65536;
+                    const int xr = (int)ceilf(sqrtf((float)rem)) + 2;
                     const int wb = (wmod(rz + iz - 1 - sz, ez_) * ey_ + wmod(ry + iy - 1 - sy, ey_)) * ex_;
                     const int ua = s_wmap[wb + w0], ub = s_wmap[wb + w1], uc = s_wmap[wb + w2];
                     if (ua >= nu || ub >= nu || uc >= nu) {  // every neighbor cell was marked; guard regardless
