@@ -959,7 +959,8 @@ char* Engine::pinned(size_t n) {
     while (want < n) want *= 2;
     want = std::min(want, std::max(n, 2 * kReadBytes));
     void* p = nullptr;
-    if (hip_check(hipHostMalloc(&p, want, hipHostMallocDefault), "hipHostMalloc")) {
+    // portable: a read may come from a thread whose current device is another one
+    if (hip_check(hipHostMalloc(&p, want, hipHostMallocPortable), "hipHostMalloc")) {
         (void)hipGetLastError();  // reported here, not by the next launch's check
         return nullptr;
     }

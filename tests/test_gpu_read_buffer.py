@@ -19,11 +19,12 @@ SHIM = r"""
 static void* runtime(const char* name) {
     return dlsym(dlopen("libamdhip64.so.7", RTLD_LAZY | RTLD_NOLOAD), name);
 }
-int allocs = 0;
+int allocs = 0, last_flags = 0;
 int fail_allocs = 0;  /* allocations still to fail */
 int hipHostMalloc(void** p, size_t n, unsigned flags) {
     int (*real)(void**, size_t, unsigned) = (int (*)(void**, size_t, unsigned))runtime("hipHostMalloc");
     allocs++;
+    last_flags = flags;
     return real(p, fail_allocs > 0 && fail_allocs-- ? (size_t)1 << 60 : n, flags);
 }
 static void* volatile launched = 0;  /* the stream of a graph launch not waited for yet */
@@ -91,6 +92,19 @@ except fmd.FmdError as x:
 e.step(s, 5)
 p, v, im = e.state(s)         # there is memory again
 assert np.isfinite(p).all() and e.steps_done(s) == 10
+e.close()
+print("ok")
+""")
+
+
+def test_the_buffer_is_of_every_device(tmp_path):
+    """A thread that reads an engine may have another device current (the flag is
+    hipHostMallocPortable)."""
+    _run(tmp_path, r"""
+e = fmd.Engine(0)
+s = e.add(desc(300))
+e.state(s)
+assert var("allocs").value == 1 and var("last_flags").value & 1
 e.close()
 print("ok")
 """)
