@@ -44,7 +44,11 @@ int size_class(int natoms);
 // 43.8 / 38.7, 20,000 42.9 / 41.4, 24,000 46.0 / 47.5, 40,000 45.1 / 52.9;
 // 48 replicas of 1,000 to 6,000 beads 79.2 / 70.2.  (Four kernels, 1.5 us less,
 // since k_rank moves the atoms; the crossing stays between 16,000 and 24,000.)
+// Batches of more replicas than CUs, which take the workgroups in rounds, gain
+// too (against the five kernels and list build of before: 512 x 1,000 beads
+// 101.8 / 80.7, 1,024 x 4,000 568.8 / 488.5, 512 x 16,000 1,003 / 885).
 constexpr int kSortInDecide = 20480;
+static_assert(kSortInDecide <= 65535, "16-bit counts and first slots");
 
 // Readback goes through pinned host memory, this many atoms at a time.
 constexpr int kReadAtoms = 1 << 17;
@@ -82,7 +86,7 @@ struct Batch {
     bool fork = false;        // the step builds lists beside the force pass (launch_step_seq)
     bool fork_known = false;
     int64_t steps_since_fork = 0;  // steps launched since that choice
-    bool wgsort = false;      // every replica's cell sort may run in one workgroup
+    bool wgsort = false;      // every replica's cell keys fit the sort by one workgroup
     int max_atoms = 0;        // of one replica
     std::vector<int> ord;     // host copy of d_reps
     void* block = nullptr;    // the arrays above, carved from one device block

@@ -744,7 +744,7 @@ Batch* Engine::batch_for(const std::vector<int>& ids_in) {
         b->any_tab = b->any_tab || reps_[id]->desc.ntables > 0;
         b->max_keys = std::max(b->max_keys, reps_[id]->desc.ncell_cap);
         b->max_atoms = std::max(b->max_atoms, reps_[id]->natoms);
-        b->wgsort = b->wgsort && reps_[id]->desc.ncell_cap <= kWgSortKeys && reps_[id]->natoms <= kWgSortAtoms;
+        b->wgsort = b->wgsort && reps_[id]->desc.ncell_cap <= kWgSortKeys;
     }
     if (ord.size() > (size_t)kMaxReplicas) {
         delete b;

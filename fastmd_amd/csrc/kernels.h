@@ -25,17 +25,15 @@ struct Launch {
     hipStream_t stream;
 };
 
-// Limits of the cell sort by one workgroup: cell keys (64 KiB of LDS) and atoms
-// (16-bit slots).
+// Cell keys that the sort by one workgroup holds the counts of (64 KiB of LDS).
 constexpr int kWgSortKeys = 32768;
-constexpr int kWgSortAtoms = 65535;
 
 enum BoundaryMode { BND_PRIME = 0, BND_STEP = 1, BND_START = 2, BND_REDUCE = 3 };
 enum ControlOp { CTL_RUN = 0, CTL_FORCE_REBUILD = 1 };
 
 void launch_pre(const Launch& l);
 // The rebuild decision of every replica; with `sort` (every replica within
-// kWgSortKeys and kWgSortAtoms) also the cell sort of those that rebuild, after
+// kWgSortKeys and kSortInDecide) also the cell sort of those that rebuild, after
 // which only the list build is left of the rebuild phases.
 void launch_decide(const Launch& l, bool sort);
 // The rebuild phases (Morton cell sort and, if `build`, the Verlet lists) of

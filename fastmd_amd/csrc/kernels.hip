@@ -118,7 +118,7 @@ template <class T> __device__ inline const FMD_GLOBAL T* gview(const T* p) {
 // store's trip to memory; a global store does not.
 template <class T> __device__ inline FMD_GLOBAL T* gmut(T* p) { return (FMD_GLOBAL T*)p; }
 
-constexpr int kMaxBlockK = 256;  // launch bound of k_build and k_force
+constexpr int kMaxBlockK = 256;  // launch bound of k_force
 constexpr int kLJChunk = 8;      // neighbors per software-pipelined chunk (kcap % 8 == 0)
 constexpr int kLJTail = 4;       // rows are padded to multiples of this; a last chunk may be this short
 constexpr int kBuildChunk = 8;   // list-build candidates whose loads are issued together
@@ -361,10 +361,10 @@ __global__ void __launch_bounds__(256) k_pre(const RepDesc* __restrict__ descs,
 // ---------------------------------------------------------------------------
 // The Morton-ordered cell sort (below, k_bin to k_rank) of one replica by one
 // workgroup of 1024 threads: the same order, in one kernel and with the cell
-// counts in LDS, two 16-bit counts a word (at most kWgSortKeys cell keys and
-// kWgSortAtoms atoms).  One CU moves the replica's state, so its time grows with
-// the atoms, while five kernels cost their launches on every step, rebuilding
-// or not (1.5 us each).
+// counts in LDS, two 16-bit counts a word (at most kWgSortKeys cell keys; the
+// engine lets it sort kSortInDecide atoms at most).  One CU moves the replica's
+// state, so its time grows with the atoms, while the four kernels cost their
+// launches on every step, rebuilding or not (1.5 us each).
 // ---------------------------------------------------------------------------
 constexpr int kSortThreads = 1024;
 constexpr int kWgSortNear = 16384;
@@ -655,7 +655,8 @@ __global__ void k_control(const RepDesc* __restrict__ descs, const int* __restri
 // Morton-ordered cell sort.  Cells have side >= rc+skin on the reference grid;
 // the cell key is the 3-D Morton interleave of the cell coordinates, so the
 // slot order is a Morton curve over cells, and within a cell atoms are ordered
-// by global id (deterministic).
+// by their grid coordinate along x, then global id (deterministic; the list
+// build searches a cell's atoms by x).
 // ---------------------------------------------------------------------------
 // The rebuild kernels walk the batch's compact list of rebuilding tiles
 // (k_rebuild_list), so their cost follows the replicas that rebuild.
@@ -1065,10 +1066,14 @@ constexpr int kColWords = 18;  // words a row in the placement by columns
 // each tile's nine rows of cells are shared out over its SPLIT waves (part
 // w / kGroupTiles), which keeps the order of the entries.
 //
-// What bounds it: instruction issue with every CU holding four groups (of a
-// group's 119 us in a 1M-bead melt the scan takes 37, the placement 28, the
-// bonded tables 11, the window and union 20), and one group's latency when
-// fewer groups than CUs are built (52 us).  Masks instead of appending each hit
+// What bounds it: the groups' chains of dependent LDS reads, compares and
+// barriers.  With every CU holding four groups (1M beads) the waves still wait
+// 62% of their time, VALU instructions are issued in 59% of the cycles, and HBM
+// moves 1.4 GB in 460 us, 65% of the copy rate; with one group a slot (a step of
+// staggered replicas) VALU issue is 35%, and where fewer groups than CUs are
+// built it is one group's latency (52 us).  Of a group's 119 us at 1M beads the
+// scan takes 37, the placement 28, the bonded tables 11, the window and union
+// 20.  Masks instead of appending each hit
 // as it is found: the rows are written once, whole 128-byte rows at a time
 // (appended, each lane's 2-byte stores fell in a row of their own, and the
 // rows were then read back and moved: 165 us a group), and the parts of a
@@ -2888,8 +2893,8 @@ void launch_control(const Launch& l, int op, int64_t arg) {
     if (l.nr <= 0) return;
     k_control<<<cdiv(l.nr, 64), 64, 0, l.stream>>>(l.descs, l.reps, l.nr, op, arg);
 }
-// k_build and k_force are compiled for at most kMaxBlock threads per block;
-// any other request runs at the default shape.
+// k_force is compiled for at most kMaxBlock threads per block; any other request
+// runs at the default shape.
 static constexpr int kMaxBlock = kMaxBlockK;
 static inline int valid_block(int b) { return (b == 64 || b == 128 || b == 256) ? b : kMaxBlock; }
 
